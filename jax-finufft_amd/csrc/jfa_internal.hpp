@@ -107,6 +107,18 @@ template <typename T>
 int launch_fft_twiddles(int64_t n, T *tw, hipStream_t stream);
 template <typename T>
 int launch_fft_lds(T *data, int64_t n, int64_t batch, const T *tw, int sign, hipStream_t stream);
+// Stages of one axis of the pruned FFT passes (fft_axis.hip): length L (2, 3, 5
+// -smooth, at most 4096) as `count` radices, P = L / the smallest of them
+// threads per transform.  False where those passes cannot run an axis.
+struct AxisFft {
+    int L, P, count;
+    int r[8];
+    int t[8];  // first entry of stage s's twiddles (s >= 1), ntw of them in all
+    int ntw;
+};
+bool axis_fft(int64_t L, size_t real_size, AxisFft *f);
+template <typename T>
+int launch_axis_twiddles(const AxisFft &f, T *tw, hipStream_t s);
 // Held around every rocFFT plan creation and destruction: calls from several
 // host threads (concurrent transforms through the plan cache) are serialised
 // there rather than relying on the library's own locking.

@@ -469,6 +469,24 @@ extern "C" void jfa_default_opts(jfa_opts *o) {
 
 extern "C" const char *jfa_last_error(void) { return jfa::last_error(); }
 
+// Stages and twiddles of every axis for the one-kernel-per-axis FFT passes;
+// plans with an axis those passes cannot run keep axis_ok = false (rocFFT).
+static int setup_axis_fft(jfa_plan p) {
+    const size_t real = p->is_double ? 8 : 4;
+    for (int d = 0; d < p->dim; ++d)
+        if (!axis_fft(p->geom.nf[d], real, &p->axis[d])) return JFA_OK;
+    for (int d = 0; d < p->dim; ++d) {
+        const AxisFft &f = p->axis[d];
+        JFA_HIP_CHECK(hipMalloc(&p->d_tw[d], 2 * real * std::max(f.ntw, 1)));
+        const int rc = p->is_double ? launch_axis_twiddles<double>(f, (double *)p->d_tw[d], p->stream)
+                                    : launch_axis_twiddles<float>(f, (float *)p->d_tw[d], p->stream);
+        if (rc) return rc;
+    }
+    p->used = true;  // work on p->stream
+    p->axis_ok = true;
+    return JFA_OK;
+}
+
 // Fill the kernel tables (Horner coefficients and per-dimension 1/psi_hat) for
 // a grid geometry that is already set.
 int jfa::upload_kernel_tables(jfa_plan p, const int64_t *nmodes_for_dk) {
@@ -606,6 +624,12 @@ extern "C" int jfa_makeplan(int type, int dim, const int64_t *nmodes, int iflag,
         if (rc) {
             jfa_destroy(p);
             return rc;
+        }
+        if (!o.gpu_spreadinterponly && dim > 1) {
+            if (int rc2 = setup_axis_fft(p)) {
+                jfa_destroy(p);
+                return rc2;
+            }
         }
         if (!o.gpu_spreadinterponly) {
             const size_t bytes = (size_t)p->batch * p->F * 2 * (p->is_double ? 8 : 4);
@@ -923,7 +947,10 @@ template <typename T>
 static int modes_to_grid(jfa_plan p, const T *fk, T *fw, int nb, StageTimer &tm) {
     const GridGeom &g = p->geom;
     int rc;
-    if (fft_is_pruned(p)) {
+    if (p->axis_ok) {
+        if ((rc = reserve_fwt(p))) return rc;
+        if ((rc = axis_modes_to_grid<T>(p, fk, (T *)p->d_fwt, fw, nb))) return rc;
+    } else if (fft_is_pruned(p)) {
         if ((rc = pruned_amplify<T>(p, fk, fw, nb))) return rc;
         tm.mark("amplify");
         if ((rc = pruned_modes_fft<T>(p, fw, nb))) return rc;
@@ -980,6 +1007,12 @@ int jfa::execute_12(jfa_plan p, T *c, T *fk) {
                 tm.mark("zero");
             }
             if ((rc = spread_timed<T>(p, cb, M, fw, p->F, nb, tm.on ? &tm : nullptr))) return rc;
+            if (p->axis_ok) {
+                if ((rc = reserve_fwt(p))) return rc;
+                if ((rc = axis_grid_to_modes<T>(p, fw, (T *)p->d_fwt, fb, nb))) return rc;
+                tm.mark("fft");
+                continue;
+            }
             if (fft_is_pruned(p)) {
                 if ((rc = pruned_grid_fft<T>(p, fw, nb))) return rc;
                 tm.mark("fft");
@@ -1132,6 +1165,7 @@ extern "C" int jfa_destroy(jfa_plan p) {
         for (auto &kv : p->fft1_plans) rocfft_plan_destroy(kv.second);
     }
     free_ptr(p->d_fwt);
+    for (auto &d : p->d_tw) free_ptr(d);
     if (p->fft_info) rocfft_execution_info_destroy(p->fft_info);
     free_ptr(p->d_fft_work);
     free_ptr(p->d_coef);

@@ -47,6 +47,10 @@ struct jfa_plan_s {
     // rocFFT
     std::map<int, rocfft_plan> fft_plans;  // by batch count
     std::map<std::pair<int64_t, int64_t>, rocfft_plan> fft1_plans;  // 1D, by (length, batch)
+    // pruned FFT passes (fft_axis.hip) where every axis supports them
+    bool axis_ok = false;
+    jfa::AxisFft axis[3] = {};
+    void *d_tw[3] = {nullptr, nullptr, nullptr};  // twiddles, by axis
     void *d_fwt = nullptr;             // compact buffer of the pruned 2D / 3D FFT
     size_t fwt_bytes = 0;
     rocfft_execution_info fft_info = nullptr;
@@ -122,6 +126,14 @@ template <typename T>
 int pruned_amplify(jfa_plan p, const T *fk, T *fw, int nb);
 template <typename T>
 int pruned_modes_fft(jfa_plan p, T *fw, int nb);
+// The same between the grid fw and the modes fk in one pass per axis, scaling
+// included (fft_axis.hip; plans with axis_ok), through a work buffer of n0 x nf1
+// (x nf2) values per transform.
+int reserve_fwt(jfa_plan p);
+template <typename T>
+int axis_grid_to_modes(jfa_plan p, T *fw, T *work, T *fk, int nb);
+template <typename T>
+int axis_modes_to_grid(jfa_plan p, const T *fk, T *work, T *fw, int nb);
 bool strip_applicable(jfa_plan p);
 int setup_strip(jfa_plan p);
 int upload_kernel_tables(jfa_plan p, const int64_t *nmodes_for_dk);
