@@ -213,21 +213,25 @@ struct BinIndex {
     int maxsub;
 };
 
-// Scratch of the point sort: keys/values for the radix sort and its temp.
+// Scratch of the point sort: the keys before and after, and radix_temp_bytes of
+// scratch.
 struct SortScratch {
     unsigned *key_in, *key_out;
     void *temp;
-    size_t temp_bytes;
-    // 0, 1, 2, ... (at least as many as keys sorted), or nullptr: the values
-    // of sorts with an odd number of passes, which would otherwise copy the
-    // keys and materialise the indices before their first pass
-    const unsigned *iota = nullptr;
 };
-// iota[i] = i for i < n
-int launch_iota(unsigned *iota, int64_t n, hipStream_t stream);
+// Stable sort of kin[0 .. M) by bits [b0, b1) (bits above b1 are zero): sorted
+// keys to kout, their input positions to vout.  Where one workgroup holds all
+// keys and the bins are few it also writes bin_start (see bin_bounds_kernel)
+// and sets *bounded.  temp: radix_temp_bytes(M, b1 - b0), or of more keys.
+constexpr int kWidestSortBits = 22;  // the span with the largest scratch
+size_t radix_temp_bytes(int64_t M, int bits = kWidestSortBits);
+int radix_sort(void *temp, const unsigned *kin, unsigned *kout, unsigned *vout, int64_t M,
+               int b0, int b1, int64_t nbins, int bin_shift, int *bin_start, bool *bounded,
+               hipStream_t stream);
+// Bits the strip sorts order by, for nbins (strip, row) bins.
+int strip_sort_bits(int64_t nbins);
 
 // Launchers (kernels_*.hip).  All queue work on `stream` and return a JFA code.
-size_t sort_temp_bytes(int64_t M);
 // Bin, radix-sort and gather M points: idx/l0/tv in bin order, bin_start
 // (nbins + 1) and, when sub_start is non-null, the LDS-subproblem prefix
 // (sub_start holds nbins + 1 + 2 * ceil(nbins / 256) + 1 ints: the prefix, then

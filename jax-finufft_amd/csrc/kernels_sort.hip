@@ -3,9 +3,9 @@
 // lib/kernels.cc.cu:63-68; device code absent from the reference).
 //
 //   1. keys:   key[j] = bin of point j (from its first tap)
-//   2. sort:   rocPRIM radix sort of (key, j) pairs over the bits the bin
-//              count needs, the values j from a counting iterator (no
-//              atomics, so clustered inputs cost the same)
+//   2. sort:   stable radix sort of (key, j) pairs over the bits the bin count
+//              needs (radix.hip; no data-dependent order or cost, so clustered
+//              inputs cost the same)
 //   3. bounds: bin_start[b] = first sorted position with key >= b (binary
 //              search per bin), and for the LDS method the subproblem prefix
 //   4. gather: for sorted position p, j = idx[p]: write the point's wrapped
@@ -20,9 +20,6 @@
 // The bin of a point and the tap window the spreader uses both come from
 // fold_point() on the coordinate in double, so they agree exactly.
 #include <algorithm>
-
-#include <rocprim/device/device_radix_sort.hpp>
-#include <rocprim/iterator/counting_iterator.hpp>
 
 #include "jfa_device.hpp"
 
@@ -506,76 +503,7 @@ int key_bits(int64_t nbins) {
     return bits;
 }
 
-// Onesweep with 10-bit digits.  A span of 9-10 key bits then takes one pass,
-// and 17-20 (25-30) bits two (three), where 8-bit digits take two, three (four):
-// 1e7 (key, index) pairs over 20 bits sort in 182 us instead of 303 us on
-// MI355X, with the same (stable) result.
-using TenBitDigits = rocprim::radix_sort_config<
-    rocprim::default_config, rocprim::default_config,
-    rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 16>,
-                                        rocprim::kernel_config<1024, 8>, 10,
-                                        rocprim::block_radix_rank_algorithm::match>>;
-
-// 11-bit digits for spans of 11 bits (one pass) and 21-22 bits (two passes
-// instead of three; 1e7 pairs over 20 bits: 246 us with 11-bit digits against
-// 303 us with 8-bit).
-using ElevenBitDigits = rocprim::radix_sort_config<
-    rocprim::default_config, rocprim::default_config,
-    rocprim::radix_sort_onesweep_config<rocprim::kernel_config<1024, 16>,
-                                        rocprim::kernel_config<1024, 16>, 11,
-                                        rocprim::block_radix_rank_algorithm::match>>;
-
-// Sorts (key, index) pairs; the indices 0, 1, ... come from a counting
-// iterator, so no kernel writes them and the first pass does not read them.
-template <typename V>
-hipError_t sort_pairs_with(void *temp, size_t &bytes, const unsigned *kin, unsigned *kout, V vin,
-                           unsigned *vout, unsigned M, int b0, int b1, int digits,
-                           hipStream_t stream) {
-    if (digits == 10)
-        return rocprim::radix_sort_pairs<TenBitDigits>(temp, bytes, kin, kout, vin, vout, M, b0,
-                                                       b1, stream);
-    if (digits == 11)
-        return rocprim::radix_sort_pairs<ElevenBitDigits>(temp, bytes, kin, kout, vin, vout, M,
-                                                          b0, b1, stream);
-    return rocprim::radix_sort_pairs(temp, bytes, kin, kout, vin, vout, M, b0, b1, stream);
-}
-
-// Digit width for a span of key bits (see the configurations above).
-int digit_bits(int bits) {
-    if ((bits > 8 && bits <= 10) || (bits > 16 && bits <= 20) || (bits > 24 && bits <= 30))
-        return 10;
-    if (bits == 11 || (bits > 20 && bits <= 22)) return 11;
-    return 8;
-}
-
-// With an odd number of passes the first pass writes the output buffers, and
-// rocPRIM first copies keys and values to its temporary buffers unless it can
-// tell that they do not alias the output, which it cannot for a counting
-// iterator; those sorts read their values from `iota` when there is one.
-hipError_t sort_pairs(void *temp, size_t &bytes, const unsigned *kin, unsigned *kout,
-                      unsigned *vout, unsigned M, int b0, int b1, hipStream_t stream,
-                      const unsigned *iota = nullptr) {
-    const int digits = digit_bits(b1 - b0);
-    const int passes = (b1 - b0 + digits - 1) / digits;
-    if (iota && passes % 2 == 1)
-        return sort_pairs_with(temp, bytes, kin, kout, iota, vout, M, b0, b1, digits, stream);
-    return sort_pairs_with(temp, bytes, kin, kout, rocprim::counting_iterator<unsigned>(0u), vout,
-                           M, b0, b1, digits, stream);
-}
-
-__global__ void __launch_bounds__(256) iota_kernel(unsigned *iota, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) iota[i] = (unsigned)i;
-}
-
 }  // namespace
-
-int launch_iota(unsigned *iota, int64_t n, hipStream_t stream) {
-    if (n <= 0) return JFA_OK;
-    iota_kernel<<<(unsigned)((n + 255) / 256), 256, 0, stream>>>(iota, n);
-    JFA_HIP_CHECK(hipGetLastError());
-    return JFA_OK;
-}
 
 int launch_fill_zero(void *p, int64_t bytes, hipStream_t stream) {
     if (bytes <= 0) return JFA_OK;
@@ -594,43 +522,16 @@ int launch_fill_zero(void *p, int64_t bytes, hipStream_t stream) {
     return JFA_OK;
 }
 
-size_t sort_temp_bytes(int64_t M) {
-    size_t bytes = 0, bytes10 = 0, bytes11 = 0;
-    const unsigned *k = nullptr;
-    unsigned *ko = nullptr;
-    const rocprim::counting_iterator<unsigned> vi(0u);
-    const unsigned n = (unsigned)(M > 0 ? M : 1);
-    if (rocprim::radix_sort_pairs(nullptr, bytes, k, ko, vi, ko, n, 0, 32, (hipStream_t)0) !=
-            hipSuccess ||
-        rocprim::radix_sort_pairs<TenBitDigits>(nullptr, bytes10, k, ko, vi, ko, n, 0, 30,
-                                                (hipStream_t)0) != hipSuccess ||
-        rocprim::radix_sort_pairs<ElevenBitDigits>(nullptr, bytes11, k, ko, vi, ko, n, 0, 22,
-                                                   (hipStream_t)0) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    // the same sorts with the values read from an index array
-    size_t pb = 0, pb10 = 0, pb11 = 0;
-    const unsigned *vp = nullptr;
-    if (rocprim::radix_sort_pairs(nullptr, pb, k, ko, vp, ko, n, 0, 32, (hipStream_t)0) !=
-            hipSuccess ||
-        rocprim::radix_sort_pairs<TenBitDigits>(nullptr, pb10, k, ko, vp, ko, n, 0, 30,
-                                                (hipStream_t)0) != hipSuccess ||
-        rocprim::radix_sort_pairs<ElevenBitDigits>(nullptr, pb11, k, ko, vp, ko, n, 0, 22,
-                                                   (hipStream_t)0) != hipSuccess) {
-        (void)hipGetLastError();
-        return 0;
-    }
-    return std::max({bytes, bytes10, bytes11, pb, pb10, pb11});
-}
-
-// bin_start from the sorted keys and, with sub_start, the subproblem prefix
+// bin_start from the sorted keys (unless the sort wrote it) and, with sub_start, the subproblem prefix
 // (block sums of the large form live after the nbins + 1 prefix entries).
 static int bins_and_subproblems(const GridGeom &g, int64_t M, const unsigned *skey, int *bin_start,
-                         int *sub_start, int *nsub, int maxsub, hipStream_t stream) {
-    const unsigned blocks = (unsigned)((g.nbins + 1 + 255) / 256);
-    bin_bounds_kernel<<<blocks, 256, 0, stream>>>(M, g.nbins, g.keyshift, skey, bin_start);
-    JFA_HIP_CHECK(hipGetLastError());
+                         bool bounded, int *sub_start, int *nsub, int maxsub,
+                         hipStream_t stream) {
+    if (!bounded) {
+        const unsigned blocks = (unsigned)((g.nbins + 1 + 255) / 256);
+        bin_bounds_kernel<<<blocks, 256, 0, stream>>>(M, g.nbins, g.keyshift, skey, bin_start);
+        JFA_HIP_CHECK(hipGetLastError());
+    }
     if (sub_start && g.nbins <= kSmallBins) {
         subs_small_kernel<<<1, 1024, 0, stream>>>((int)g.nbins, bin_start, maxsub, sub_start,
                                                   nsub);
@@ -650,6 +551,7 @@ template <typename T>
 int launch_sort_points(const GridGeom &g, int64_t M, const T *x, const T *y, const T *z,
                        const SortScratch &s, int *bin_start, int *sub_start, int *nsub,
                        int maxsub, int *idx, int *l0, T *tv, hipStream_t stream) {
+    bool bounded = false;
     if (M > 0) {
         if (aligned4<T>(g.dim, x, y, z, s.key_in, s.key_in)) {
             const unsigned blocks = (unsigned)((M + 1023) / 1024);
@@ -662,13 +564,13 @@ int launch_sort_points(const GridGeom &g, int64_t M, const T *x, const T *y, con
                                         g, M, x, y, z, s.key_in));
         }
         JFA_HIP_CHECK(hipGetLastError());
-        size_t bytes = s.temp_bytes;
-        JFA_HIP_CHECK(sort_pairs(s.temp, bytes, s.key_in, s.key_out,
-                                 (unsigned *)idx, (unsigned)M, 0,
-                                 key_bits(g.nbins) + g.keyshift, stream, s.iota));
+        if (int rc = radix_sort(s.temp, s.key_in, s.key_out, (unsigned *)idx, M, 0,
+                                key_bits(g.nbins) + g.keyshift, g.nbins, g.keyshift, bin_start,
+                                &bounded, stream))
+            return rc;
     }
-    if (int rc = bins_and_subproblems(g, M, s.key_out, bin_start, sub_start, nsub, maxsub,
-                                      stream))
+    if (int rc = bins_and_subproblems(g, M, s.key_out, bin_start, bounded, sub_start, nsub,
+                                      maxsub, stream))
         return rc;
     if (M > 0) {
         const unsigned blocks = (unsigned)((M + 255) / 256);
@@ -683,6 +585,7 @@ template <typename T>
 int launch_sort_points_keyed(const GridGeom &g, int64_t M, const T *x, const T *y, const T *z,
                              const SortScratch &s, int *bin_start, int *sub_start, int *nsub,
                              int maxsub, int *idx, T *rec, hipStream_t stream) {
+    bool bounded = false;
     if (M > 0) {
         if (aligned4<T>(g.dim, x, y, z, s.key_in, rec)) {
             const unsigned blocks = (unsigned)((M + 1023) / 1024);
@@ -696,13 +599,13 @@ int launch_sort_points_keyed(const GridGeom &g, int64_t M, const T *x, const T *
         }
         JFA_HIP_CHECK(hipGetLastError());
         // only the bin bits are sorted; the offset bits ride along
-        size_t bytes = s.temp_bytes;
-        JFA_HIP_CHECK(sort_pairs(s.temp, bytes, s.key_in, s.key_out,
-                                 (unsigned *)idx, (unsigned)M, g.keyshift,
-                                 g.keyshift + key_bits(g.nbins), stream, s.iota));
+        if (int rc = radix_sort(s.temp, s.key_in, s.key_out, (unsigned *)idx, M, g.keyshift,
+                                g.keyshift + key_bits(g.nbins), g.nbins, g.keyshift, bin_start,
+                                &bounded, stream))
+            return rc;
     }
-    if (int rc = bins_and_subproblems(g, M, s.key_out, bin_start, sub_start, nsub, maxsub,
-                                      stream))
+    if (int rc = bins_and_subproblems(g, M, s.key_out, bin_start, bounded, sub_start, nsub,
+                                      maxsub, stream))
         return rc;
     return JFA_OK;
 }
@@ -724,14 +627,17 @@ int launch_fold_points(const GridGeom &g, int64_t M, const T *x, const T *y, con
 // matter, so the three lowest key bits are left out of the (stable) sort.
 constexpr int kStripSortLowBit = 3;
 
+int strip_sort_bits(int64_t nbins) { return key_bits(nbins) + kStripKeyShift - kStripSortLowBit; }
+
 int sort_strip_keys(int64_t M, int64_t nbins, const SortScratch &s, int *bin_start, int *idx,
                     hipStream_t stream) {
-    if (M > 0) {
-        size_t bytes = s.temp_bytes;
-        JFA_HIP_CHECK(sort_pairs(s.temp, bytes, s.key_in, s.key_out,
-                                 (unsigned *)idx, (unsigned)M, kStripSortLowBit,
-                                 key_bits(nbins) + kStripKeyShift, stream, s.iota));
-    }
+    bool bounded = false;
+    if (M > 0)
+        if (int rc = radix_sort(s.temp, s.key_in, s.key_out, (unsigned *)idx, M,
+                                kStripSortLowBit, key_bits(nbins) + kStripKeyShift, nbins,
+                                kStripKeyShift, bin_start, &bounded, stream))
+            return rc;
+    if (bounded) return JFA_OK;
     const unsigned blocks = (unsigned)((nbins + 1 + 255) / 256);
     bin_bounds_kernel<<<blocks, 256, 0, stream>>>(M, nbins, kStripKeyShift, s.key_out,
                                                   bin_start);

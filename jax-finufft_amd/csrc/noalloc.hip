@@ -103,7 +103,6 @@ __global__ void __launch_bounds__(256)
 struct Buffers {
     unsigned *key_in, *key_out;
     void *sort_temp;
-    size_t sort_temp_bytes;
     int *idx, *bin_start, *piece_start, *npieces, *piece_unit, *heavy, *blocksum;
     float *rec, *pack, *tiles, *fw, *G, *tw0, *tw1, *coef, *dk0, *dk1;
     int64_t tile_stride;
@@ -116,8 +115,6 @@ Buffers carve(Carve &c, const StripGeom &sg, const GridGeom &g, int64_t M, int64
     b.key_in = c.take<unsigned>(4 * m);
     b.key_out = c.take<unsigned>(4 * m);
     b.idx = c.take<int>(4 * m);
-    b.sort_temp_bytes = sort_temp_bytes(m);
-    b.sort_temp = c.take<unsigned char>(b.sort_temp_bytes);
     b.rec = c.take<float>(8 * m);
     b.pack = c.take<float>(16 * m);
     b.bin_start = c.take<int>(4 * (g.nbins + 1));
@@ -128,6 +125,12 @@ Buffers carve(Carve &c, const StripGeom &sg, const GridGeom &g, int64_t M, int64
     b.blocksum = c.take<int>(4 * (2 * ((sg.nunits + 255) / 256) + 2));
     b.tile_stride = strip_max_pieces(sg, M) * strip_tile_cells(sg);
     b.tiles = c.take<float>(8 * b.tile_stride);
+    // the sort is done before the tiles are written: its scratch lives there
+    // where it fits
+    const size_t sort_bytes = radix_temp_bytes(m, strip_sort_bits(g.nbins));
+    b.sort_temp = sort_bytes <= (size_t)(8 * b.tile_stride)
+                      ? (void *)b.tiles
+                      : (void *)c.take<unsigned char>(sort_bytes);
     b.fw = c.take<float>(8 * g.nf[0] * g.nf[1]);
     b.G = c.take<float>(8 * n0 * g.nf[1]);
     b.tw0 = c.take<float>(8 * g.nf[0]);
@@ -225,7 +228,7 @@ int run_noalloc(jfa_stream_t stream_, float eps, int64_t iflag, int64_t n_tot, i
     const int sign = iflag >= 0 ? 1 : -1;
     const int kem = gpu_kerevalmeth ? 1 : 0;
     const int64_t Ntot = n0 * n1, F = g.nf[0] * g.nf[1];
-    const SortScratch ss{b.key_in, b.key_out, b.sort_temp, b.sort_temp_bytes};
+    const SortScratch ss{b.key_in, b.key_out, b.sort_temp};
     const StripPts<float> pts{n_j, b.idx, b.key_out, b.pack, nullptr, nullptr, 0, 0, 0};
     for (int64_t idx = 0; idx < n_tot; ++idx) {
         // the reference's offsets (lib/kernels.cc.cu:57-60)

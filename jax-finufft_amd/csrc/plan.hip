@@ -684,22 +684,15 @@ int jfa::reserve_points(jfa_plan p, int64_t M) {
     }
     if (M > p->cap_M) {
         for (void **q : {(void **)&p->d_idx, (void **)&p->d_l0, (void **)&p->d_key_in,
-                         (void **)&p->d_key_out, (void **)&p->d_iota, &p->d_t, &p->d_sort_temp})
+                         (void **)&p->d_key_out, &p->d_t, &p->d_sort_temp})
             free_ptr(*q);
         const int64_t cap = std::max<int64_t>(M, 1);
         JFA_HIP_CHECK(hipMalloc(&p->d_idx, sizeof(int) * cap));
-        JFA_HIP_CHECK(hipMalloc(&p->d_iota, sizeof(unsigned) * cap));
-        if (int rc = launch_iota(p->d_iota, cap, p->stream)) return rc;
         JFA_HIP_CHECK(hipMalloc(&p->d_l0, sizeof(int) * cap * p->dim));
         JFA_HIP_CHECK(hipMalloc(&p->d_key_in, sizeof(unsigned) * cap));
         JFA_HIP_CHECK(hipMalloc(&p->d_key_out, sizeof(unsigned) * cap));
         JFA_HIP_CHECK(hipMalloc(&p->d_t, real * cap * p->dim));
-        p->sort_temp_bytes = sort_temp_bytes(cap);
-        if (!p->sort_temp_bytes) {
-            set_error("radix sort temp size query failed");
-            return JFA_ERR_HIP;
-        }
-        JFA_HIP_CHECK(hipMalloc(&p->d_sort_temp, p->sort_temp_bytes));
+        JFA_HIP_CHECK(hipMalloc(&p->d_sort_temp, radix_temp_bytes(cap)));
         p->cap_M = cap;
     }
     return JFA_OK;
@@ -750,8 +743,7 @@ static int sort_points(jfa_plan p, int64_t M, const T *x, const T *y, const T *z
     GridGeom &g = p->geom;
     p->keyed = false;
     if (p->method == JFA_METHOD_STRIP) {
-        SortScratch s{p->d_key_in, p->d_key_out, p->d_sort_temp, p->sort_temp_bytes,
-                      p->d_iota};
+        SortScratch s{p->d_key_in, p->d_key_out, p->d_sort_temp};
         if (p->dim == 3)
             return launch_sort_points_slices<T>(g, p->sg.S, M, x, y, z, s, p->d_bin_start,
                                                 p->d_idx, (T *)p->d_t, p->stream);
@@ -761,7 +753,7 @@ static int sort_points(jfa_plan p, int64_t M, const T *x, const T *y, const T *z
     const bool sorted = p->method == JFA_METHOD_SM || p->opts.gpu_sort;
     if (!sorted)
         return launch_fold_points<T>(g, M, x, y, z, p->d_idx, p->d_l0, (T *)p->d_t, p->stream);
-    SortScratch s{p->d_key_in, p->d_key_out, p->d_sort_temp, p->sort_temp_bytes, p->d_iota};
+    SortScratch s{p->d_key_in, p->d_key_out, p->d_sort_temp};
     if (keyed_bins(g)) {
         p->keyed = true;
         return launch_sort_points_keyed<T>(g, M, x, y, z, s, p->d_bin_start,
@@ -1172,7 +1164,7 @@ extern "C" int jfa_destroy(jfa_plan p) {
     for (auto &d : p->d_dk) free_ptr(d);
     free_ptr(p->d_fw);
     for (void **q : {(void **)&p->d_idx, (void **)&p->d_l0, (void **)&p->d_key_in,
-                     (void **)&p->d_key_out, (void **)&p->d_iota, &p->d_sort_temp, &p->d_t,
+                     (void **)&p->d_key_out, &p->d_sort_temp, &p->d_t,
                      (void **)&p->d_bin_start, (void **)&p->d_sub_start, (void **)&p->d_nsub,
                      (void **)&p->d_piece_start, (void **)&p->d_npieces,
                      (void **)&p->d_piece_unit, (void **)&p->d_heavy,

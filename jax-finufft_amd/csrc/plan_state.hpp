@@ -62,9 +62,7 @@ struct jfa_plan_s {
     int *d_idx = nullptr, *d_l0 = nullptr;
     void *d_t = nullptr;
     unsigned *d_key_in = nullptr, *d_key_out = nullptr;  // radix sort
-    unsigned *d_iota = nullptr;        // 0, 1, ..., cap_M - 1 (values of odd-pass sorts)
     void *d_sort_temp = nullptr;
-    size_t sort_temp_bytes = 0;
     int *d_bin_start = nullptr, *d_sub_start = nullptr, *d_nsub = nullptr;
 
     // 2D strip spreader

@@ -57,7 +57,6 @@ struct jfa_ragged_s {
     void *d_t = nullptr;
     unsigned *d_key_in = nullptr, *d_key_out = nullptr;
     void *d_sort_temp = nullptr;
-    size_t sort_temp_bytes = 0;
     int *d_bin_start = nullptr, *d_piece_start = nullptr, *d_npieces = nullptr,
         *d_piece_unit = nullptr, *d_heavy = nullptr,
         *d_blocksum = nullptr;
@@ -421,12 +420,7 @@ int allocate(jfa_ragged r) {
     JFA_HIP_CHECK(hipMalloc(&r->d_t, real * cap * 2));
     JFA_HIP_CHECK(hipMalloc(&r->d_key_in, sizeof(unsigned) * cap));
     JFA_HIP_CHECK(hipMalloc(&r->d_key_out, sizeof(unsigned) * cap));
-    r->sort_temp_bytes = sort_temp_bytes(cap);
-    if (!r->sort_temp_bytes) {
-        set_error("radix sort temp size query failed");
-        return JFA_ERR_HIP;
-    }
-    JFA_HIP_CHECK(hipMalloc(&r->d_sort_temp, r->sort_temp_bytes));
+    JFA_HIP_CHECK(hipMalloc(&r->d_sort_temp, radix_temp_bytes(cap)));
     JFA_HIP_CHECK(hipMalloc(&r->d_bin_start, sizeof(int) * (r->rl.nbins + 1)));
     JFA_HIP_CHECK(hipMalloc(&r->d_piece_start, sizeof(int) * (r->rl.nunits + 1)));
     JFA_HIP_CHECK(hipMalloc(&r->d_npieces, sizeof(int) * 4));
@@ -552,7 +546,7 @@ int enqueue_execute(jfa_ragged r, hipStream_t s) {
 
 template <typename T>
 int run_t(jfa_ragged r, hipStream_t s) {
-    SortScratch ss{r->d_key_in, r->d_key_out, r->d_sort_temp, r->sort_temp_bytes};
+    SortScratch ss{r->d_key_in, r->d_key_out, r->d_sort_temp};
     if (int rc = launch_ragged_sort<T>(r->rl, ss, r->d_idx, (T *)r->d_t, s)) return rc;
     if (!r->use_graph || r->graph_state < 0) return enqueue_execute<T>(r, s);
     if (r->graph_state == 0) {
