@@ -76,6 +76,8 @@ struct StripGeom {
     int pmax;       // most points per piece (a unit has ceil(count / pmax) pieces)
 };
 
+constexpr int kStripPiece = 4096;  // default pmax
+
 // Complex cells of one piece's scratch tile, and the most pieces M points can
 // make (sum over units of ceil(count / pmax) <= units + M / pmax).
 inline int64_t strip_tile_cells(const StripGeom &sg) { return (int64_t)(sg.H + sg.ns - 1) * 64; }

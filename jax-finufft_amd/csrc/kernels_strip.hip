@@ -476,7 +476,7 @@ __device__ __forceinline__ int left_windows(int w, int step, int span, int n, in
 template <typename T, int NS>
 __device__ __forceinline__ void merge_unit(const StripGeom &sg, const int *__restrict__ piece_start,
                                            const T *__restrict__ scratch, T *__restrict__ fw,
-                                           int u) {
+                                           int u, int reduced) {
     constexpr int SW = 65 - NS;
     const int sz = u / sg.K, k = u - sz * sg.K;  // strip over all slices, unit row
     const int z = sz / sg.S, s = sz - z * sg.S;  // slice, strip within it
@@ -503,8 +503,9 @@ __device__ __forceinline__ void merge_unit(const StripGeom &sg, const int *__res
             if (i < ncs && j < nck) {
                 const int u2 = (z * sg.S + cs[i]) * sg.K + ck[j];
                 pfirst[3 * i + j] = piece_start[u2] - base;
-                // a crowded unit's pieces were summed into its first tile
-                pcount[3 * i + j] = min(piece_start[u2 + 1] - piece_start[u2], 1);
+                // reduced: a crowded unit's pieces were summed into its first tile
+                const int np = piece_start[u2 + 1] - piece_start[u2];
+                pcount[3 * i + j] = reduced ? min(np, 1) : np;
             }
         }
     const int c = threadIdx.x & (kStripLanes - 1);
@@ -636,9 +637,9 @@ template <typename T, int NS>
 __global__ void __launch_bounds__(256)
     strip_merge_kernel(StripGeom sg, const int *__restrict__ piece_start,
                        const T *__restrict__ scratch, int64_t scratch_stride, T *__restrict__ fw,
-                       int64_t fw_stride) {
+                       int64_t fw_stride, int reduced) {
     merge_unit<T, NS>(sg, piece_start, scratch + 2 * scratch_stride * blockIdx.y,
-                      fw + 2 * fw_stride * blockIdx.y, (int)blockIdx.x);
+                      fw + 2 * fw_stride * blockIdx.y, (int)blockIdx.x, reduced);
 }
 
 // Piece table of one plan's units in three launches (counts with per-block
@@ -650,6 +651,15 @@ __global__ void __launch_bounds__(256)
 __global__ void __launch_bounds__(1024)
     strip_units_blocks_kernel(int nu, int nblk, const int *__restrict__ blocksum, int *blockoff,
                               int *piece_start, int *npieces, int *heavy);
+// The same in one launch of one workgroup, for few units.
+constexpr int kSmallUnits = 4096;
+__global__ void __launch_bounds__(1024)
+    strip_units_small_kernel(StripGeom sg, const int *__restrict__ bin_start, int *piece_start,
+                             int *npieces, int *piece_unit, int *heavy) {
+    piece_scan(
+        sg.nunits, [&](int u) { return unit_pieces(sg, bin_start, u); }, piece_start, npieces,
+        piece_unit, heavy);
+}
 __global__ void __launch_bounds__(256)
     strip_units_scan_kernel(int nu, const int *__restrict__ blockoff, int *piece_start,
                             int *piece_unit, int *heavy);
@@ -861,10 +871,14 @@ __global__ void __launch_bounds__(256)
     const int v = unit_virt[gu];
     const RaggedVirt d = virt[v];
     merge_unit<T, NS>(d.sg, piece_start + d.unit_off, scratch_all + 2 * d.tile_off,
-                      fw_all + 2 * d.fw_off, gu - d.unit_off);
+                      fw_all + 2 * d.fw_off, gu - d.unit_off, 1);
 }
 
 }  // namespace
+
+// A launch of strip_reduce_kernel is worth about this many pieces read in series
+// by one merge workgroup.
+constexpr int kMergePieces = 16;
 
 template <typename T>
 int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *bin_start,
@@ -874,7 +888,13 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
                         int64_t fw_stride, T *scratch, int64_t scratch_stride, int ntr,
                         int phases, hipStream_t stream) {
     if (ntr == 0 || pts.M == 0) return JFA_OK;
-    if (phases & kStripUnits) {
+    if ((phases & kStripUnits) && sg.nunits <= kSmallUnits) {
+        // 24 units (4000-point call): 3 launches 8.8 us, one 3.6 us; 9216 units:
+        // 13.1 against 15.9 us
+        strip_units_small_kernel<<<1, 1024, 0, stream>>>(sg, bin_start, piece_start, npieces,
+                                                         piece_unit, heavy);
+        JFA_HIP_CHECK(hipGetLastError());
+    } else if (phases & kStripUnits) {
         const unsigned nblk = (unsigned)((sg.nunits + 255) / 256);
         int *blockoff = blocksum + nblk;  // nblk + 1 entries
         strip_units_count_kernel<<<nblk, 256, 0, stream>>>(sg, bin_start, piece_start, blocksum);
@@ -894,7 +914,9 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
             spread_strip_kernel<T, NS_><<<dim3(grid, ntr), kStripLanes, 0, stream>>>(
                 sg, pts, bin_start, piece_start, npieces, piece_unit, coef, b, kerevalmeth,
                 pack_stride, scratch, scratch_stride);
-        if (phases & kStripMerge) {
+        // few pieces in all: the merge sums a crowded unit's itself
+        const int reduced = pts.M / sg.pmax > kMergePieces;
+        if ((phases & kStripMerge) && reduced) {
             const int64_t rb = strip_max_heavy(sg, pts.M) *
                                ((strip_tile_cells(sg) + 255) / 256);
             strip_reduce_kernel<T, NS_>
@@ -905,7 +927,7 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
             // two waves per unit: units are 8 rows or more (256 threads: 0.044 vs
             // 0.0415 ms at the 2048^2 bench size, 0.063 vs 0.056 ms clustered)
             strip_merge_kernel<T, NS_><<<dim3((unsigned)sg.nunits, ntr), 128, 0, stream>>>(
-                    sg, piece_start, scratch, scratch_stride, fw, fw_stride);
+                    sg, piece_start, scratch, scratch_stride, fw, fw_stride, reduced);
     });
     JFA_HIP_CHECK(hipGetLastError());
     return JFA_OK;

@@ -213,7 +213,7 @@ jfa::StripGeom jfa::strip_geometry(GridGeom &g, int pmax, int min_h, int rows) {
     sg.H = (int)H;
     sg.K = (int)((g.nf[1] + H - 1) / H);
     sg.nunits = sg.nz * sg.S * sg.K;
-    sg.pmax = pmax > 0 ? pmax : 4096;
+    sg.pmax = pmax > 0 ? pmax : kStripPiece;
     // bins: (slice, strip, exact row), rows fastest
     g.bs[0] = sg.SW;
     g.bs[1] = 1;
@@ -669,6 +669,35 @@ int jfa::default_maxsub(jfa_plan p) {
     return p->type == 2 && p->dim < 3 ? 4096 : 1024;
 }
 
+// Subproblem and piece sizes for M points, unless the caller chose one.
+//
+// LDS subproblems: the full size (default_maxsub) once that many bins or chunks
+// fill the GPU; with under 512 of them, M / 2048 points, never below the 256
+// lanes of a workgroup (30,011 fp64 points on 2048 cells, 1D interpolation:
+// 8 workgroups 187 us, 118 workgroups 7 us).  Splitting where there are enough
+// only reloads tiles: 1e7 points in 1024 bins of 64 x 64, halves instead of
+// whole bins, 0.265 -> 0.367 ms.
+//
+// Strip pieces: a wave walks its piece in series, so one crowded unit in full
+// pieces can outlast the rest of the launch.  Units are split above twice the
+// mean unit, and above a wave slot's share of the points of all nb transforms
+// (300,007 centre-dense points, 4 transforms, 640 x 512: spreading 168 us in pieces of
+// 4096, 65 us by this rule); evenly filled units stay whole, since every
+// extra piece writes a tile and is summed again (4e6 uniform points on 1024^2
+// in halves: 121 -> 137 us, and 10 us of reduction).
+static void size_chunks(jfa_plan p, int64_t M) {
+    if (p->opts.gpu_maxsubprobsize > 0) return;
+    auto chunk = [](int64_t v, int64_t most) {
+        return (int)std::min(most, std::max<int64_t>(256, (v + 63) / 64 * 64));
+    };
+    const int full = default_maxsub(p);
+    p->maxsub = std::max(p->geom.nbins, M / full) < 512 ? chunk(M / 2048, full) : full;
+    if (p->method == JFA_METHOD_STRIP) {
+        const int64_t Mq = p->dim == 3 ? M * p->geom.ns : M;
+        p->sg.pmax = chunk(std::max(2 * Mq / p->sg.nunits, Mq * p->batch / 4096), kStripPiece);
+    }
+}
+
 // Grow the point-dependent scratch to hold M points.
 int jfa::reserve_points(jfa_plan p, int64_t M) {
     const size_t real = p->is_double ? 8 : 4;
@@ -815,6 +844,7 @@ int jfa::setpts_12(jfa_plan p, int64_t M, const void *x, const void *y, const vo
     if (rc) return rc;
     p->M = M;
     if (M == 0) return JFA_OK;
+    size_chunks(p, M);
     if (p->is_double)
         return sort_points<double>(p, M, (const double *)x, (const double *)y,
                                    (const double *)z);

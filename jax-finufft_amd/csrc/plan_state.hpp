@@ -22,7 +22,7 @@ struct jfa_plan_s {
                                      // at setpts from the point density
     bool keyed = false;              // sorted points without a gather: d_key_out + d_t
                                      // (point-major), see SortedPts
-    int maxsub = 4096;
+    int maxsub = 4096;               // most points per LDS subproblem on the current points
     hipStream_t stream = nullptr;
     int device = 0;
     bool used = false;                 // work has been queued on `stream`
