@@ -49,8 +49,8 @@ __device__ __forceinline__ Folded fold_point(double x, int64_t nf, double scale,
 // polynomial P_i at -t.  Writing P_i(t) = E(t^2) + t O(t^2) (its even and odd
 // coefficients), both taps come from one Horner pass over E and O in t^2:
 // about NC + 2 FMAs per pair instead of 2 (NC - 1).
-template <typename T, int NS, bool HORNER>
-__device__ __forceinline__ void eval_kernel(const T *__restrict__ coef, T beta, T t, T *ker) {
+template <typename T, int NS, bool HORNER, typename Coef>
+__device__ __forceinline__ void eval_kernel(Coef coef, T beta, T t, T *ker) {
     if constexpr (HORNER) {
         constexpr int NC = horner_nc(NS);
         constexpr int NE = (NC + 1) / 2, NO = NC / 2;  // even / odd coefficient counts

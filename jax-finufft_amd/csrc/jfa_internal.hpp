@@ -87,12 +87,12 @@ inline int64_t strip_max_pieces(const StripGeom &sg, int64_t M) {
 // Units with more than one piece hold more than pmax points each.
 inline int64_t strip_max_heavy(const StripGeom &sg, int64_t M) { return M / (sg.pmax + 1) + 1; }
 
-// Strip geometry for a 2D grid g (nf and ns set): units of H rows sized for
-// about 4096 units, at least min_h rows, H in [ns, nf1 - ns + 1] so that a
-// cell is covered by at most two units per axis; also sets g's bins to
-// (strip, row), rows fastest.
-// rows > 0 sets the unit height instead (gpu_binsizey), within the same clamp.
-StripGeom strip_geometry(GridGeom &g, int pmax, int min_h, int rows = 0);
+// Rows of the spreading kernel's accumulators, in tiles of 16: a unit's H +
+// ns - 1 rows fit them.
+constexpr int strip_row_tiles(int ns) { return ns <= 8 ? 1 : 2; }
+// Strip geometry for a grid g (nf and ns set), with units of H rows; also sets
+// g's bins to (strip, row), rows fastest.  rows > 0 asks for lower units.
+StripGeom strip_geometry(GridGeom &g, int pmax, int rows = 0);
 int ensure_rocfft();
 
 // Batched 1D FFTs in LDS (fft_lds.hip), for rows of length n = 2^a 3^b 5^c <=
@@ -193,6 +193,9 @@ struct SortedPts {
 // gather.  key = (bin << kStripKeyShift) | X with bin = bin_off + s*nf1 + l0y
 // (s the strip) and X = l0x - s*SW in [0, SW).
 constexpr int kStripKeyShift = 6;
+// Lowest key bit the strip sorts order by: points of a (strip, row) bin keep
+// input order (the spreader groups each batch by column itself).
+constexpr int kStripSortLowBit = kStripKeyShift;
 template <typename T>
 struct StripPts {
     int64_t M;

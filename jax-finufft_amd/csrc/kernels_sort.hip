@@ -621,12 +621,8 @@ int launch_fold_points(const GridGeom &g, int64_t M, const T *x, const T *y, con
     return JFA_OK;
 }
 
-// Shared tail of the strip sorts: radix sort of (key, index) and bin bounds.
-// The strip spreaders need the points of a strip in row order and, within a
-// row, grouped by 8-column block (X >> 3); the order within a block does not
-// matter, so the three lowest key bits are left out of the (stable) sort.
-constexpr int kStripSortLowBit = 3;
-
+// Shared tail of the strip sorts: radix sort of (key, index) by (strip, row), and
+// bin bounds.
 int strip_sort_bits(int64_t nbins) { return key_bits(nbins) + kStripKeyShift - kStripSortLowBit; }
 
 int sort_strip_keys(int64_t M, int64_t nbins, const SortScratch &s, int *bin_start, int *idx,

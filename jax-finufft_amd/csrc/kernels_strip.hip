@@ -10,23 +10,23 @@
 // columns; strip s owns points whose first x-tap l0x lies in
 // [s*SW, (s+1)*SW), so all of their taps fall in the 64 columns
 // [s*SW, s*SW + 64).  Points are sorted by (strip, l0y) (the "y-major" bins
-// set up by the plan; for ns <= 8 also by 8-column block within the row), so
-// within a strip they arrive in row order.  A strip is cut into units of H
-// consecutive l0y rows, and one wave spreads one unit.
+// set up by the plan).  A strip is cut into units of H consecutive l0y rows.
+// A unit's whole tile, 16 or 32 rows x 64 columns, lives in the registers of the
+// wave that spreads it, as the accumulators of MFMA products.
 //
-// ns <= 8 (strip8_piece): cells are assigned to lanes modulo 8 in both
-// directions, so that every lane does useful work for every point (below).
-// Wider kernels (wide_piece): lane x owns column s*SW + x and holds a rolling
-// window of ns rows (real and imaginary parts) in registers.  Points are staged
-// 64 at a time: each lane evaluates one point's ns x-weights and ns y-weights
-// (Horner) and writes the x-weights and c*y-weights to wave-private LDS; then
-// the wave walks the batch in order, every lane reading its own x-weight (zero
-// outside the point's window) and the point's y-weights by broadcast, and doing
-// 2*ns FMAs into its window.  When the next point starts a later row, the
-// window's first row is complete and is written out.  No atomics touch LDS.
+// Spreading is a contraction over points: tile[y][x] += sum_p (c_p ky_p[y])
+// kx_p[x].  strip_piece takes four points at a time as the K dimension of a
+// 16 x 16 x 4 MFMA, whose 16 rows are the tile's and whose 16 columns are a
+// frame of the tile, one product for the real and one for the imaginary part
+// (details there).  Points are staged 64 at a time: each lane evaluates one
+// point's ns x-weights and ns y-weights (Horner) and writes them to
+// wave-private LDS in frame order.  No atomics touch LDS.
+//
+// Bound by instruction issue, VALU and MFMA together (a SIMD issues one or the
+// other): figures at strip_piece.
 //
 // Output.  A unit's points are cut into pieces of at most `pmax` points (an
-// empty unit has none), one wave per piece.  A piece writes its rows with plain
+// empty unit has none), one workgroup of one or four waves per piece.  A piece writes its rows with plain
 // coalesced stores into its own scratch tile of (H + ns - 1) x 64 cells; a
 // merge kernel then writes every fine-grid cell once, as the sum over the
 // units covering it (one to four, up to nine next to a narrow last strip or
@@ -45,12 +45,24 @@
 // strip, row), so the strips of all slices form one list of nz * S strips
 // (strip index z * S + s) and the 2D bodies run unchanged.  Only the merge
 // needs the slice: its neighbours are taken within the slice.
+#include <utility>
+
 #include "jfa_device.hpp"
 
 namespace jfa {
 namespace {
 
 constexpr int kStripLanes = 64;
+
+// f(integral_constant 0), ..., f(integral_constant N - 1)
+template <typename F, int... Is>
+__device__ __forceinline__ void unroll_seq(F &&f, std::integer_sequence<int, Is...>) {
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void unroll(F &&f) {
+    unroll_seq(f, std::make_integer_sequence<int, N>{});
+}
 
 template <typename T>
 struct alignas(2 * sizeof(T)) Pair {
@@ -61,36 +73,101 @@ struct alignas(4 * sizeof(T)) Quad {
     T x, y, z, w;
 };
 
-// Pairs per staged point in the ns <= 8 layout: 8 and one pad.  Each lane
-// writes its own point's pairs, so the point stride is the lane stride of the
-// staging writes; 9 pairs (18 or 36 dwords, twice an odd number) put the
-// lanes of one write on distinct banks, where 8 pairs would put every fourth
-// (64 banks) or second (32 banks) lane on the same bank.
-constexpr int kPointPairs = 9;
+// MFMA 16 x 16 x 4: D[i][j] += sum_k A[i][k] B[k][j].  Lane l holds A[l % 16][l / 16],
+// B[l / 16][l % 16] and D[row(r, l / 16)][l % 16], r < 4.
+template <typename T>
+struct Mfma;
+template <>
+struct Mfma<float> {
+    typedef float Acc __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ Acc mul(float a, float b, Acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int r, int g) { return 4 * g + r; }
+};
+template <>
+struct Mfma<double> {
+    typedef double Acc __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ Acc mul(double a, double b, Acc c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int r, int g) { return 4 * r + g; }
+};
 
-// LDS staging of one wave: ns <= 8 uses the weight pairs (and c * y-weights
-// for NT transforms at once), wider kernels the column weights and c *
-// y-weights per point.
-template <typename T, int NS, int NT = 1, bool MOD8 = (NS <= 8)>
-struct StripLds;
-template <typename T, int NS, int NT>
-struct StripLds<T, NS, NT, true> {
-    // per point q, lane column a: (weight in block bx, in bx + 1)
-    Pair<T> w[kStripLanes * kPointPairs];
-    // per transform, point q, row offset dy: c * ky[dy]
-    Pair<T> cky[NT][kStripLanes * kPointPairs];
-};
-// ns > 8: the point stride is rounded up to an odd number of values for the
-// same reason.
+// Shape of a unit's tile in MFMA terms (see strip_piece).
 template <int NS>
-constexpr int wide_stride() { return NS | 1; }
-template <typename T, int NS, int NT>
-struct StripLds<T, NS, NT, false> {
-    T kx[kStripLanes * wide_stride<NS>()];
-    T cky[kStripLanes * wide_stride<NS>() * 2];
-    int lx[kStripLanes];
-    int ly[kStripLanes];
+struct StripShape {
+    static constexpr bool kNarrow = NS <= 8;
+    static constexpr int kRowTiles = strip_row_tiles(NS);  // of 16 rows
+    // narrow: frames start every 8 columns, so one 16-column frame holds a
+    // point's taps; wide: every 16 columns, a point reaches into the next frame
+    static constexpr int kFrames = kNarrow ? 8 : 4;
+    static constexpr int kFrameShift = kNarrow ? 3 : 4;
+    // Values per staged point and axis.  Narrow: the weights, then zeros, so that
+    // any 16-value window that starts up to 8 before a point's weights (units
+    // are at most 9 rows) reads zeros around them (the previous point's zeros lie
+    // in front).  Wide: the
+    // weights alone.  Odd, so that the points of one write are on distinct banks.
+    static constexpr int kStride = kNarrow ? 17 : NS | 1;
+    static constexpr int kGuard = kNarrow ? 8 : 0;  // zeros before the first point
+    static constexpr int kValues = kGuard + kStripLanes * kStride - (kNarrow ? 1 : 0);
+    // Slots of a batch: every frame's points rounded up to groups of four, and a
+    // group read ahead.
+    static constexpr int kSlots = kStripLanes + 3 * kFrames + 4;
 };
+
+// A staged point as the MFMA loop finds it: the strengths of NT transforms, and
+// two 16-bit values that locate its y (high) and x weights.
+template <typename T, int NT>
+struct alignas(16) StripSlot {
+    Pair<T> c[NT];
+    unsigned at;
+};
+
+// LDS staging of one wave: the weights by point of the batch, the points by slot.
+// (ns <= 8 in fp32: 10,232 bytes, so that 16 waves share a CU's 160 KiB.)
+template <typename T, int NS, int NT = 1>
+struct StripLds {
+    StripSlot<T, NT> slot[StripShape<NS>::kSlots];
+    T ky[StripShape<NS>::kValues];
+    T kx[StripShape<NS>::kValues];
+};
+
+// The ns weights of a point along one axis to LDS.  Doubles a few taps at a time:
+// all chains at once need more registers than the accumulators leave.
+template <typename T, int NS, typename Coef>
+__device__ __forceinline__ void stage_weights(Coef coef, T beta, int horner, T t, T *out) {
+    if (sizeof(T) == 8 && NS > 8 && horner) {
+        constexpr int NC = horner_nc(NS), NE = (NC + 1) / 2, NO = NC / 2;  // as in eval_kernel
+        const T s = t * t;
+        unroll<(NS + 1) / 2>([&](auto ic) {
+            constexpr int i = decltype(ic)::value;
+            T e = coef[2 * (NE - 1) * NS + i], o = coef[(2 * NO - 1) * NS + i];
+#pragma unroll
+            for (int k = NE - 2; k >= 0; --k) e = fma(e, s, coef[2 * k * NS + i]);
+#pragma unroll
+            for (int k = NO - 2; k >= 0; --k) o = fma(o, s, coef[(2 * k + 1) * NS + i]);
+            out[i] = fma(t, o, e);
+            if constexpr (NS - 1 - i != i) out[NS - 1 - i] = fma(-t, o, e);
+            if constexpr (i % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        });
+        return;
+    }
+    T k[NS];
+    if (horner)
+        eval_kernel<T, NS, true>(coef, beta, t, k);
+    else
+        eval_kernel<T, NS, false>(coef, beta, t, k);
+#pragma unroll
+    for (int i = 0; i < NS; ++i) out[i] = k[i];
+}
+
+// Order of one wave's LDS accesses: its instructions reach LDS in program order,
+// so only the compiler has to keep it.
+__device__ __forceinline__ void wave_sync() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
 
 // Strength and Horner pair of input point P: from the packed record, or from
 // the strengths (by index within the problem) and the setpts pairs (by P).
@@ -122,189 +199,70 @@ __device__ __forceinline__ PieceRange piece_range(const StripGeom &sg,
     return pr;
 }
 
-// ------------------------------------------------------------ ns > 8 body
-
-template <typename T, int NS, typename Lds>
-__device__ __forceinline__ void wide_piece(const StripGeom &sg, const StripPts<T> &pts,
-                                           const int *__restrict__ bin_start, int u, int sub,
-                                           const T *__restrict__ coef, T beta, int horner,
-                                           T *__restrict__ tile, Lds &lds) {
-    constexpr int NSP = wide_stride<NS>();
-    const int lane = threadIdx.x;
-    const int rows_tile = sg.H + NS - 1;
+// ------------------------------------------------------------ one piece
+//
+// Spreads one piece's points for NT transforms sharing them: transform k's
+// strengths at pts.c + k * pts.c_tstride (NT = 1 may read packed records instead),
+// its tile at tile + k * tile_tstride.
+//
+// The accumulators hold the unit's tile: rows r0 .. r0 + 16 kRowTiles - 1 by
+// frames of 16 columns.  ns <= 8: eight frames 8 columns apart, one row tile, so a
+// point adds to exactly one frame: one MFMA each for the real and imaginary parts
+// of four points (half the columns are zeros).  ns > 8: four frames, two row
+// tiles; a point adds to its frame and the next, and to both row tiles where its
+// rows straddle them (batches are in row order, so a row tile no point of the
+// batch touches is skipped).  Each MFMA's four points must share a frame: the
+// points of a batch are ranked by frame (one ballot per bit of the frame) and
+// listed in that order in the slots, every frame's list filled up to a multiple of
+// four with zero strengths; the weights stay where the point's lane wrote them.
+//
+// Counted at 1e7 uniform points on 2048^2 (fp32, ns = 8), per point: 19 MFMA
+// cycles, 7.3 VALU wave instructions (of 4 cycles; 104 Horner FMAs over 64 lanes,
+// ranking, operand addresses), 7 LDS cycles.  263 us, where adding one point after
+// another to per-lane windows of the tile (10.4 VALU instructions and 9.6 LDS cycles
+// per point) took 268; a unit's points now need no order within a row, which makes
+// the sort's keys 3 bits shorter.  The walk was a chain of LDS reads and adds, so
+// smaller and wider problems gain more: 1e6 fp64 points on 1024^2 at ns = 11 275 ->
+// 185 us, 300,007 points x 3 transforms on 501 x 333 at ns = 6 65 -> 46, 100,000
+// points on 256^2 29 -> 11; 1e6 points and as many targets of a 3D type 3 at ns = 8
+// 507 -> 314.
+//
+// W waves share a piece: each spreads a run of its points into accumulators of its
+// own, which are added through LDS in wave order at the end.
+template <typename T, int NS, int NT, int W>
+__device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<T> &pts,
+                                            const int *__restrict__ bin_start, int u, int sub,
+                                            const T *__restrict__ coef, T beta, int horner,
+                                            T *__restrict__ tile, int64_t tile_tstride,
+                                            StripLds<T, NS, NT> *lds_all) {
+    using Sh = StripShape<NS>;
+    using M = Mfma<T>;
+    using Acc = typename M::Acc;
+    constexpr int RT = Sh::kRowTiles, NF = Sh::kFrames, S = Sh::kStride;
+    const int lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+    const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+    StripLds<T, NS, NT> &lds = lds_all[wave];
     const PieceRange pr = piece_range(sg, bin_start, u, sub);
-    const int r0 = pr.r0, pb = pr.pb, pe = pr.pe;
+    const int r0 = pr.r0;
+    // this wave's points: whole batches, as even as they come
+    const int per = ((pr.pe - pr.pb + W - 1) / W + kStripLanes - 1) & -kStripLanes;
+    const int pb = min(pr.pb + wave * per, pr.pe), pe = min(pb + per, pr.pe);
     // key >> kStripKeyShift = rowbase + l0y for every point of this strip
     const int64_t rowbase = pts.bin_off + (int64_t)(u / sg.K) * sg.nf1;
-    T acc_r[NS], acc_i[NS];
+    Acc re[NT][RT][NF], im[NT][RT][NF];
+    unroll<NT * RT * NF>([&](auto c) {
+        constexpr int e = decltype(c)::value, t = e / (RT * NF), h = e / NF % RT, f = e % NF;
+        re[t][h][f] = im[t][h][f] = Acc{0, 0, 0, 0};
+    });
+    // the weights' places before any is staged: zeros, as around them later
+    for (int e = lane; e < Sh::kValues; e += kStripLanes) lds.ky[e] = lds.kx[e] = T(0);
+    StripSlot<T, NT> none;
 #pragma unroll
-    for (int b = 0; b < NS; ++b) acc_r[b] = acc_i[b] = T(0);
-    // rolling window: acc[b] holds row rcur + b
-    int rcur = r0;
-    auto flush = [&](int row) {
-        {
-            const int64_t q = (int64_t)(row - r0) * kStripLanes + lane;
-            tile[2 * q] = acc_r[0];
-            tile[2 * q + 1] = acc_i[0];
-        }
-#pragma unroll
-        for (int b = 0; b + 1 < NS; ++b) {
-            acc_r[b] = acc_r[b + 1];
-            acc_i[b] = acc_i[b + 1];
-        }
-        acc_r[NS - 1] = acc_i[NS - 1] = T(0);
-    };
-    for (int bb = pb; bb < pe; bb += kStripLanes) {
-        const int nb = min(kStripLanes, pe - bb);
-        // stage: lane q evaluates point bb + q
-        if (lane < nb) {
-            const int p = bb + lane;
-            const unsigned key = pts.key[p];
-            const Quad<T> rq = point_record(pts, pts.idx[p]);
-            const T cr = rq.x, ci = rq.y;
-            const Pair<T> tt{rq.z, rq.w};
-            T kx[NS], ky[NS];
-            if (horner) {
-                eval_kernel<T, NS, true>(coef, beta, tt.x, kx);
-                eval_kernel<T, NS, true>(coef, beta, tt.y, ky);
-            } else {
-                eval_kernel<T, NS, false>(coef, beta, tt.x, kx);
-                eval_kernel<T, NS, false>(coef, beta, tt.y, ky);
-            }
-#pragma unroll
-            for (int a = 0; a < NS; ++a) lds.kx[lane * NSP + a] = kx[a];
-#pragma unroll
-            for (int b = 0; b < NS; ++b) {
-                lds.cky[(lane * NSP + b) * 2] = cr * ky[b];
-                lds.cky[(lane * NSP + b) * 2 + 1] = ci * ky[b];
-            }
-            lds.lx[lane] = (int)(key & ((1u << kStripKeyShift) - 1));
-            lds.ly[lane] = (int)((key >> kStripKeyShift) - rowbase);
-        }
-        __syncthreads();
-        for (int q = 0; q < nb; ++q) {
-            const int ly = lds.ly[q];
-            while (rcur < ly) {
-                flush(rcur);
-                ++rcur;
-            }
-            const int kk = lane - lds.lx[q];
-            const bool in = kk >= 0 && kk < NS;
-            const T kxv = in ? lds.kx[q * NSP + (in ? kk : 0)] : T(0);
-            const T *cy = &lds.cky[q * NSP * 2];
-#pragma unroll
-            for (int b = 0; b < NS; ++b) {
-                acc_r[b] = fma(cy[2 * b], kxv, acc_r[b]);
-                acc_i[b] = fma(cy[2 * b + 1], kxv, acc_i[b]);
-            }
-        }
-        __syncthreads();
-    }
-    // drain the window and every remaining row of the tile
-    const int rstop = r0 + rows_tile;
-    while (rcur < rstop) {
-        flush(rcur);
-        ++rcur;
-    }
-}
-
-// ------------------------------------------------------------ ns <= 8 body
-//
-// Points are staged 64 at a time in wave-private LDS: per point q, its
-// x-weights placed in a 16-column frame starting at the 8-column block
-// bx = X >> 3 of its first tap X (frame column c = (X & 7) + i holds kx[i];
-// stored as pairs by c & 7: (weight at c, weight at c + 8)), and its
-// strength times its y-weights, c * ky[dy].  The wave then walks the batch in
-// runs of equal (row, bx): the sort key's low bits order the points by row and
-// block, so every point of a run adds into the same two column blocks of an
-// 8-row window of 64 columns held in registers (row y in window slot y & 7).
-// When a later row starts, the window's first row is complete: it is written
-// to the piece's tile and its slot cleared.
-//
-// Lane (a, r) = (lane & 7, lane >> 3) holds columns a, a+8, ..., a+56 of the
-// row in slot r.  An ns x ns footprint (ns <= 8) puts at most one cell in
-// every lane, so per point each lane adds the products of its weight pair
-// with the point's c * ky for its row into blocks bx and bx + 1.
-
-// The accumulator window (see above).
-template <typename T, int NT>
-struct Window8 {
-    T re[NT][8], im[NT][8];
-
-    __device__ __forceinline__ void clear() {
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int b = 0; b < 8; ++b) re[t][b] = im[t][b] = T(0);
-    }
-
-    // points [q0, q1) of the staged batch, all in row Y and block BX
-    template <int BX>
-    __device__ __forceinline__ void walk(const Pair<T> *__restrict__ s_w,
-                                         const Pair<T> (*__restrict__ s_cky)
-                                             [kStripLanes * kPointPairs],
-                                         int q0, int q1, int Y, int lane) {
-        const int a = lane & 7, dy = ((lane >> 3) - Y) & 7;
-#pragma unroll 4
-        for (int q = q0; q < q1; ++q) {
-            const Pair<T> w = s_w[q * kPointPairs + a];
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const Pair<T> cy = s_cky[t][q * kPointPairs + dy];
-                re[t][BX] = fma(w.x, cy.x, re[t][BX]);
-                im[t][BX] = fma(w.x, cy.y, im[t][BX]);
-                if constexpr (BX < 7) {  // block 8 would only receive zero weights
-                    re[t][BX + 1] = fma(w.y, cy.x, re[t][BX + 1]);
-                    im[t][BX + 1] = fma(w.y, cy.y, im[t][BX + 1]);
-                }
-            }
-        }
-    }
-
-    // write window row `row` (tile row row - r0) and clear its slot
-    __device__ __forceinline__ void flush(int row, int r0, int lane, T *__restrict__ tile,
-                                          int64_t tile_tstride) {
-        if ((row & 7) != (lane >> 3)) return;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            Pair<T> *dst = reinterpret_cast<Pair<T> *>(tile + t * tile_tstride) +
-                           (int64_t)(row - r0) * kStripLanes + (lane & 7);
-#pragma unroll
-            for (int b = 0; b < 8; ++b) dst[8 * b] = Pair<T>{re[t][b], im[t][b]};
-#pragma unroll
-            for (int b = 0; b < 8; ++b) re[t][b] = im[t][b] = T(0);
-        }
-    }
-};
-
-// One piece for NT transforms sharing the points: transform k's strengths at
-// pts.c + k * pts.c_tstride (NT = 1 may read packed records instead), its tile
-// at tile + k * tile_tstride.
-template <typename T, int NS, int NT, int LNT>
-__device__ __forceinline__ void strip8_piece(const StripGeom &sg, const StripPts<T> &pts,
-                                             const int *__restrict__ bin_start, int u, int sub,
-                                             const T *__restrict__ coef, T beta, int horner,
-                                             T *__restrict__ tile, int64_t tile_tstride,
-                                             StripLds<T, NS, LNT> &lds) {
-    static_assert(NS <= 8, "modular ownership needs ns <= 8");
-    static_assert(NT <= LNT, "LDS staging for NT transforms");
-    Pair<T> *s_w = lds.w;
-    Pair<T> (*s_cky)[kStripLanes * kPointPairs] = lds.cky;
-    const int lane = threadIdx.x;
-    const int rows_tile = sg.H + NS - 1;
-    const PieceRange pr = piece_range(sg, bin_start, u, sub);
-    const int r0 = pr.r0, pb = pr.pb, pe = pr.pe;
-    // key >> kStripKeyShift = rowbase + l0y for every point of this strip
-    const int64_t rowbase = pts.bin_off + (int64_t)(u / sg.K) * sg.nf1;
-    Window8<T, NT> win;
-    win.clear();
-    // the window holds rows R .. R+7
-    int R = r0;
+    for (int t = 0; t < NT; ++t) none.c[t] = Pair<T>{T(0), T(0)};
+    none.at = Sh::kNarrow ? (unsigned)(Sh::kGuard * sizeof(T)) * 0x10001u : 0u;
     // Software pipeline over 64-point batches: while one batch is staged and
-    // walked, the next batch's records (and other transforms' strengths) and
-    // the key and index of the batch after it are in flight.  A wave holds one
-    // unit, so without this every batch would wait for its scattered record
-    // reads with too few other waves on the SIMD to cover them.
+    // multiplied, the next batch's records (and other transforms' strengths) and
+    // the key and index of the batch after it are in flight.
     constexpr int NC = NT > 1 ? NT - 1 : 1;
     unsigned key1 = 0, key2 = 0;
     int idx1 = 0, idx2 = 0;
@@ -339,104 +297,191 @@ __device__ __forceinline__ void strip8_piece(const StripGeom &sg, const StripPts
         idx1 = idx2;
         load_record(bb + kStripLanes, idx1);
         load_index(bb + 2 * kStripLanes, key2, idx2);
-        int key = -1;  // (row << 3) | block of the lane's staged point
+        const int X = (int)(pkey & ((1u << kStripKeyShift) - 1));
+        const int Y = (int)((int64_t)(pkey >> kStripKeyShift) - rowbase) - r0;
+        // this lane's slot, and the groups of four of every frame
+        constexpr int kBits = Sh::kNarrow ? 3 : 2;
+        const unsigned frame = (unsigned)X >> Sh::kFrameShift;
+        const uint64_t in = nb < kStripLanes ? (uint64_t(1) << nb) - 1 : ~uint64_t(0);
+        uint64_t bit[kBits], same = in;
+#pragma unroll
+        for (int b = 0; b < kBits; ++b) {
+            const bool one = (frame >> b) & 1;
+            bit[b] = __ballot(one);
+            same &= one ? bit[b] : ~bit[b];
+        }
+        int groups[NF];
+        uint64_t starts = 0;  // first group of every frame, 5 bits each
+        int base = 0;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            uint64_t m = in;
+#pragma unroll
+            for (int b = 0; b < kBits; ++b) m &= (f >> b) & 1 ? bit[b] : ~bit[b];
+            starts |= (uint64_t)base << (5 * f);
+            groups[f] = (__popcll(m) + 3) >> 2;
+            base += groups[f];
+        }
+        const int slot = 4 * (int)((starts >> (5 * frame)) & 31) +
+                         (int)__builtin_amdgcn_mbcnt_hi(
+                             (unsigned)(same >> 32),
+                             __builtin_amdgcn_mbcnt_lo((unsigned)same, 0u));
+        bool low = true, high = false;
+        if constexpr (RT > 1) {
+            low = __builtin_amdgcn_readfirstlane(Y) < 16;
+            high = __builtin_amdgcn_readlane(Y, nb - 1) + NS > 16;
+        }
+        // (a wave's LDS writes land in order: the empty slots before the filled)
+        lds.slot[lane] = none;
+        if (lane + kStripLanes < Sh::kSlots) lds.slot[lane + kStripLanes] = none;
+        // opaque: hoisted out of the loop, the coefficients would not fit the scalar
+        // registers and spill; constant address space: scalar loads all the same
+        uintptr_t cf_bits = reinterpret_cast<uintptr_t>(coef);
+        asm volatile("" : "+s"(cf_bits));
+        const auto *cf = reinterpret_cast<const __attribute__((address_space(4))) T *>(cf_bits);
         if (lane < nb) {
-            const T cr = rq.x, ci = rq.y;
-            const Pair<T> tt{rq.z, rq.w};
-            const int X = (int)(pkey & ((1u << kStripKeyShift) - 1));
-            // x-weights, then y-weights: one set of ns values live at a time
-            {
-                T kx[NS];
-                if (horner)
-                    eval_kernel<T, NS, true>(coef, beta, tt.x, kx);
-                else
-                    eval_kernel<T, NS, false>(coef, beta, tt.x, kx);
-                const int ph = X & 7;
+            const int v0 = Sh::kGuard + lane * S;
+            stage_weights<T, NS>(cf, beta, horner, rq.z, lds.kx + v0);
+            stage_weights<T, NS>(cf, beta, horner, rq.w, lds.ky + v0);
+            const int ox = X & ((1 << Sh::kFrameShift) - 1);
+            StripSlot<T, NT> me;
+            me.c[0] = Pair<T>{rq.x, rq.y};
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const T v = i < NS ? kx[i] : T(0);
-                    const bool lo = ph + i < 8;
-                    s_w[lane * kPointPairs + ((ph + i) & 7)] =
-                        Pair<T>{lo ? v : T(0), lo ? T(0) : v};
+            for (int t = 1; t < NT; ++t) me.c[t] = ct[t - 1];
+            // narrow: byte offsets of where row 0 of the tile / column 0 of the frame
+            // lie in the staged values; wide: the first row, and lane and column
+            me.at = Sh::kNarrow
+                        ? (unsigned)((v0 - Y) * sizeof(T)) << 16 | (unsigned)((v0 - ox) * sizeof(T))
+                        : (unsigned)Y << 16 | (unsigned)(lane << 4) | (unsigned)ox;
+            lds.slot[slot] = me;
+        }
+        wave_sync();
+        // operands of the four points from slot 4 n: lane (i16, g) reads point g's
+        constexpr int NB = Sh::kNarrow ? 1 : 2;
+        struct Operands {
+            T y[RT], x[NB];
+            Pair<T> c[NT];
+        };
+        const StripSlot<T, NT> *next = lds.slot + g;
+        auto fetch = [&] {
+            Operands o;
+            const StripSlot<T, NT> s = *next;
+            next += 4;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) o.c[t] = s.c[t];
+            if constexpr (Sh::kNarrow) {
+                // both halves at once (neither overflows)
+                const unsigned at = s.at + (unsigned)(i16 * sizeof(T)) * 0x10001u;
+                o.y[0] = *reinterpret_cast<const T *>(
+                    reinterpret_cast<const char *>(lds.ky) + (at >> 16));
+                o.x[0] = *reinterpret_cast<const T *>(
+                    reinterpret_cast<const char *>(lds.kx) + (at & 0xffffu));
+            } else {
+                const int ya = (int)(s.at >> 16), xa = (int)(s.at & 15u);
+                const int v0 = (int)(s.at >> 4 & 63u) * S;
+#pragma unroll
+                for (int h = 0; h < RT; ++h) {
+                    const int e = i16 + 16 * h - ya;
+                    const T v = lds.ky[v0 + (unsigned(e) < NS ? e : 0)];
+                    o.y[h] = unsigned(e) < NS ? v : T(0);
+                }
+#pragma unroll
+                for (int h = 0; h < NB; ++h) {
+                    const int e = i16 + 16 * h - xa;
+                    const T v = lds.kx[v0 + (unsigned(e) < NS ? e : 0)];
+                    o.x[h] = unsigned(e) < NS ? v : T(0);
                 }
             }
-            {
-                T ky[NS];
-                if (horner)
-                    eval_kernel<T, NS, true>(coef, beta, tt.y, ky);
-                else
-                    eval_kernel<T, NS, false>(coef, beta, tt.y, ky);
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    s_cky[0][lane * kPointPairs + i] =
-                        i < NS ? Pair<T>{cr * ky[i], ci * ky[i]} : Pair<T>{T(0), T(0)};
-#pragma unroll
-                for (int t = 1; t < NT; ++t) {
-#pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        s_cky[t][lane * kPointPairs + i] =
-                            i < NS ? Pair<T>{ct[t - 1].x * ky[i], ct[t - 1].y * ky[i]}
-                                   : Pair<T>{T(0), T(0)};
-                }
+            return o;
+        };
+        Operands cur = fetch();
+        // frames as compile-time constants, so that the accumulators are separate
+        // registers to the compiler (as one array it copies it between frames)
+        unroll<NF>([&](auto fc) {
+            constexpr int f = decltype(fc)::value;
+            for (int n = groups[f]; n > 0; --n) {
+                const Operands o = cur;
+                cur = fetch();
+                unroll<RT>([&](auto hc) {
+                    constexpr int h = decltype(hc)::value;
+                    if (RT > 1 && !(h == 0 ? low : high)) return;
+                    const T y = o.y[h];
+                    unroll<NT>([&](auto tc) {
+                        constexpr int t = decltype(tc)::value;
+                        const T ar = y * o.c[t].x, ai = y * o.c[t].y;
+                        re[t][h][f] = M::mul(ar, o.x[0], re[t][h][f]);
+                        im[t][h][f] = M::mul(ai, o.x[0], im[t][h][f]);
+                        if constexpr (NB > 1 && f + 1 < NF) {
+                            // (no point of the last frame leaves it)
+                            re[t][h][f + 1] = M::mul(ar, o.x[NB - 1], re[t][h][f + 1]);
+                            im[t][h][f + 1] = M::mul(ai, o.x[NB - 1], im[t][h][f + 1]);
+                        }
+                    });
+                });
             }
-            key = ((int)((pkey >> kStripKeyShift) - rowbase) << 3) | (X >> 3);
-        }
-        const int prev = __shfl_up(key, 1);
-        const uint64_t starts = __ballot(lane < nb && (lane == 0 || key != prev));
-        __syncthreads();
-        uint64_t mask = starts;
-        while (mask) {
-            const int q0 = __builtin_ctzll(mask);
-            mask &= mask - 1;
-            const int q1 = mask ? __builtin_ctzll(mask) : nb;
-            const int gkey = __builtin_amdgcn_readlane(key, q0);
-            const int Y = gkey >> 3;
-            while (R < Y) {
-                win.flush(R, r0, lane, tile, tile_tstride);
-                ++R;
-            }
-            switch (gkey & 7) {
-                case 0: win.template walk<0>(s_w, s_cky, q0, q1, Y, lane); break;
-                case 1: win.template walk<1>(s_w, s_cky, q0, q1, Y, lane); break;
-                case 2: win.template walk<2>(s_w, s_cky, q0, q1, Y, lane); break;
-                case 3: win.template walk<3>(s_w, s_cky, q0, q1, Y, lane); break;
-                case 4: win.template walk<4>(s_w, s_cky, q0, q1, Y, lane); break;
-                case 5: win.template walk<5>(s_w, s_cky, q0, q1, Y, lane); break;
-                case 6: win.template walk<6>(s_w, s_cky, q0, q1, Y, lane); break;
-                default: win.template walk<7>(s_w, s_cky, q0, q1, Y, lane); break;
-            }
-        }
-        __syncthreads();
+        });
+        wave_sync();
     }
-    // drain the window and every remaining row of the tile
-    const int rstop = r0 + rows_tile;
-    while (R < rstop) {
-        win.flush(R, r0, lane, tile, tile_tstride);
-        ++R;
-    }
-}
-
-// One piece for nt transforms (nt <= LNT) sharing the points (see strip8_piece).
-template <typename T, int NS, int LNT>
-__device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<T> &pts,
-                                            const int *__restrict__ bin_start, int u, int sub,
-                                            const T *__restrict__ coef, T beta, int horner,
-                                            T *__restrict__ tile, int nt, int64_t tile_tstride,
-                                            StripLds<T, NS, LNT> &lds) {
-    if constexpr (NS <= 8) {
-        if (LNT > 1 && nt > 1)
-            strip8_piece<T, NS, LNT, LNT>(sg, pts, bin_start, u, sub, coef, beta, horner, tile,
-                                          tile_tstride, lds);
-        else
-            strip8_piece<T, NS, 1, LNT>(sg, pts, bin_start, u, sub, coef, beta, horner, tile,
-                                        tile_tstride, lds);
+    // the tile's rows to scratch: value e = (t, h, r, k) is row 16 h + row(r, g),
+    // column 16 k + i16 of transform t
+    const int rows_tile = sg.H + NS - 1;
+    const bool upper = i16 >= 8;
+    auto value = [&](auto ec) {
+        constexpr int e = decltype(ec)::value, t = e / (RT * 16), h = e / 16 % RT, k = e / 4 % 4,
+                      r = e % 4;
+        if constexpr (!Sh::kNarrow) {
+            return Pair<T>{re[t][h][k][r], im[t][h][k][r]};
+        } else {
+            // columns 16 k ..: the even frame 2 k, and the odd frames on either
+            // side, whose lanes are 8 columns off
+            T sr = re[t][h][2 * k + 1][r], si = im[t][h][2 * k + 1][r];
+            if constexpr (k > 0) {
+                sr = upper ? re[t][h][2 * k - 1][r] : sr;
+                si = upper ? im[t][h][2 * k - 1][r] : si;
+            } else {
+                sr = upper ? T(0) : sr;
+                si = upper ? T(0) : si;
+            }
+            return Pair<T>{re[t][h][2 * k][r] + __shfl_xor(sr, 8),
+                           im[t][h][2 * k][r] + __shfl_xor(si, 8)};
+        }
+    };
+    auto store = [&](int e, Pair<T> v) {
+        const int t = e / (RT * 16), h = e / 16 % RT, k = e / 4 % 4, r = e % 4;
+        const int row = 16 * h + M::row(r, g);
+        if (row < rows_tile)
+            reinterpret_cast<Pair<T> *>(tile + t * tile_tstride)[row * kStripLanes + 16 * k + i16] =
+                v;
+    };
+    if constexpr (W == 1) {
+        unroll<NT * RT * 16>([&](auto ec) { store(decltype(ec)::value, value(ec)); });
     } else {
-        StripPts<T> pk = pts;
-        for (int k = 0; k < nt; ++k) {
-            wide_piece<T, NS>(sg, pk, bin_start, u, sub, coef, beta, horner,
-                              tile + k * tile_tstride, lds);
-            pk.c += pts.c_tstride;
-        }
+        // eight values of every lane at a time through the staging areas; wave w
+        // adds up values w, w + W, ...
+        static_assert(sizeof(StripLds<T, NS, NT>) >= 8 * kStripLanes * sizeof(Pair<T>), "");
+        __syncthreads();
+        unroll<NT * RT * 2>([&](auto cc) {
+            constexpr int e0 = 8 * decltype(cc)::value;
+            unroll<8>([&](auto ec) {
+                constexpr int e = e0 + decltype(ec)::value;
+                reinterpret_cast<Pair<T> *>(&lds)[(e - e0) * kStripLanes + lane] =
+                    value(std::integral_constant<int, e>{});
+            });
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 8; e += W) {
+                Pair<T> v{T(0), T(0)};
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    const Pair<T> x = reinterpret_cast<const Pair<T> *>(
+                        lds_all + w)[(e + wave) * kStripLanes + lane];
+                    v.x += x.x;
+                    v.y += x.y;
+                }
+                store(e0 + e + wave, v);
+            }
+            __syncthreads();
+        });
     }
 }
 
@@ -580,24 +625,27 @@ __device__ __forceinline__ void piece_scan(int n, PiecesOf pieces, int *piece_st
 
 // ------------------------------------------------------------ one plan
 
-template <typename T, int NS>
-__global__ void __launch_bounds__(kStripLanes)
+// Waves per SIMD the spreading kernels are compiled for, by the registers of
+// their accumulators: 64 leave room for four, 128 for two, 256 for one.
+template <typename T, int NT>
+constexpr int strip_waves() { return sizeof(T) * NT == 4 ? 4 : sizeof(T) * NT == 8 ? 2 : 1; }
+
+template <typename T, int NS, int W>
+__global__ void __launch_bounds__(kStripLanes *W, (strip_waves<T, 1>()))
     spread_strip_kernel(StripGeom sg, StripPts<T> pts, const int *__restrict__ bin_start,
                         const int *__restrict__ piece_start, const int *__restrict__ npieces,
                         const int *__restrict__ piece_unit, const T *__restrict__ coef, T beta,
                         int horner, int64_t pack_stride, T *__restrict__ scratch,
                         int64_t scratch_stride) {
-    __shared__ StripLds<T, NS> lds;
+    __shared__ StripLds<T, NS> lds[W];
     pts.pack += 4 * pack_stride * blockIdx.y;
     scratch += 2 * scratch_stride * blockIdx.y;
     const int64_t tile_cells = (int64_t)(sg.H + NS - 1) * kStripLanes;
-    const int total = *npieces;
-    for (int piece = blockIdx.x; piece < total; piece += gridDim.x) {
-        const int u = piece_unit[piece];
-        const int sub = piece - piece_start[u];
-        strip_piece<T, NS>(sg, pts, bin_start, u, sub, coef, beta, horner,
-                           scratch + 2 * piece * tile_cells, 1, 0, lds);
-    }
+    const int piece = blockIdx.x;  // one workgroup per piece
+    if (piece >= *npieces) return;
+    const int u = piece_unit[piece];
+    strip_piece<T, NS, 1, W>(sg, pts, bin_start, u, piece - piece_start[u], coef, beta, horner,
+                             scratch + 2 * piece * tile_cells, 0, lds);
 }
 
 // pack[t][j] = (c[t][j], rec[j])
@@ -806,8 +854,11 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// Waves per piece.  Problems of all densities fill the GPU together: 64 problems of
+// up to 2e6 points, 1 to 8 transforms: the batch takes 4.70 ms, with four 6.03.
+constexpr int kRaggedWaves = 1;
 template <typename T, int NS>
-__global__ void __launch_bounds__(kStripLanes)
+__global__ void __launch_bounds__(kStripLanes *kRaggedWaves, (strip_waves<T, 2>()))
     ragged_strip_kernel(const RaggedVirt *__restrict__ virt, const int *__restrict__ unit_virt,
                         StripPts<T> pts, const int *__restrict__ bin_start,
                         const int *__restrict__ piece_start, const int *__restrict__ npieces,
@@ -815,24 +866,28 @@ __global__ void __launch_bounds__(kStripLanes)
                         const T *__restrict__ coef, T beta, int horner,
                         const void *const *__restrict__ ptrs, int nprob,
                         T *__restrict__ scratch_all) {
-    __shared__ StripLds<T, NS, 2> lds;
-    const int total = *npieces;
-    for (int piece = blockIdx.x; piece < total; piece += gridDim.x) {
-        const int gu = piece_unit[piece];
-        const int v = unit_virt[gu];
-        const RaggedVirt d = virt[v];
-        if (d.nt == 0) continue;  // spread together with transform t - 1
-        const int sub = piece - piece_start[gu];
-        StripPts<T> vp = pts;
-        vp.c = (const T *)ptrs[2 * nprob + d.prob] + 2 * (int64_t)d.t * d.m;
-        vp.c_tstride = 2 * d.m;
-        vp.bin_off = d.bin_off;
-        vp.idx_off = d.moff;
-        const int64_t tile_cells = (int64_t)(d.sg.H + NS - 1) * kStripLanes;
-        T *tile = scratch_all + 2 * (d.tile_off + (piece - piece_start[d.unit_off]) * tile_cells);
-        strip_piece<T, NS>(d.sg, vp, bin_start + d.bin_off, gu - d.unit_off, sub, coef, beta,
-                           horner, tile, d.nt, 2 * d.tile_next, lds);
-    }
+    __shared__ StripLds<T, NS, 2> lds[kRaggedWaves];
+    const int piece = blockIdx.x;  // one workgroup per piece
+    if (piece >= *npieces) return;
+    const int gu = piece_unit[piece];
+    const int v = unit_virt[gu];
+    const RaggedVirt d = virt[v];
+    if (d.nt == 0) return;  // spread together with transform t - 1
+    const int sub = piece - piece_start[gu];
+    StripPts<T> vp = pts;
+    vp.c = (const T *)ptrs[2 * nprob + d.prob] + 2 * (int64_t)d.t * d.m;
+    vp.c_tstride = 2 * d.m;
+    vp.bin_off = d.bin_off;
+    vp.idx_off = d.moff;
+    const int64_t tile_cells = (int64_t)(d.sg.H + NS - 1) * kStripLanes;
+    T *tile = scratch_all + 2 * (d.tile_off + (piece - piece_start[d.unit_off]) * tile_cells);
+    if (d.nt > 1)
+        strip_piece<T, NS, 2, kRaggedWaves>(d.sg, vp, bin_start + d.bin_off, gu - d.unit_off, sub,
+                                            coef, beta, horner, tile, 2 * d.tile_next, lds);
+    else
+        strip_piece<T, NS, 1, kRaggedWaves>(d.sg, vp, bin_start + d.bin_off, gu - d.unit_off, sub,
+                                            coef, beta, horner, tile, 0,
+                                            reinterpret_cast<StripLds<T, NS, 1> *>(lds));
 }
 
 // Ragged form of strip_reduce_kernel: heavy lists global units.
@@ -907,13 +962,30 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
     // one workgroup per piece (see launch_ragged_strip); 3D slice grids have
     // tens of thousands of units
     const int64_t ub = sg.nunits + pts.M / sg.pmax + 1;
-    const unsigned grid = (unsigned)(ub < (1 << 30) ? ub : (1 << 30));
+    if (ub > UINT32_MAX / kStripLanes) {  // threads of a launch
+        set_error("%lld strip pieces are too many for one launch", (long long)ub);
+        return JFA_ERR_TOO_LARGE;
+    }
+    const unsigned grid = (unsigned)ub;
+    // Waves per piece: four where an even unit has two batches of points or more
+    // (shorter waves level the last round, and few units still fill the GPU: 1e7
+    // points on 2048^2 263 us, one wave 276; 1e6 on 512^2 110, one wave 145; 300,007
+    // x 3 on 501 x 333 46, one wave 76); one in sparser units and pieces, where most
+    // of the four would find no points.
+    constexpr int kPieceWaves = 4;
+    const int waves = std::min<int64_t>(pts.M / sg.nunits, sg.pmax) >= 2 * kStripLanes &&
+                              ub <= UINT32_MAX / (kStripLanes * kPieceWaves)
+                          ? kPieceWaves
+                          : 1;
     const T b = (T)beta;
     JFA_DISPATCH_NS(sg.ns, {
-        if (phases & kStripSpread)
-            spread_strip_kernel<T, NS_><<<dim3(grid, ntr), kStripLanes, 0, stream>>>(
+        if (phases & kStripSpread) {
+            auto kernel = waves > 1 ? spread_strip_kernel<T, NS_, kPieceWaves>
+                                    : spread_strip_kernel<T, NS_, 1>;
+            kernel<<<dim3(grid, ntr), kStripLanes * waves, 0, stream>>>(
                 sg, pts, bin_start, piece_start, npieces, piece_unit, coef, b, kerevalmeth,
                 pack_stride, scratch, scratch_stride);
+        }
         // few pieces in all: the merge sums a crowded unit's itself
         const int reduced = pts.M / sg.pmax > kMergePieces;
         if ((phases & kStripMerge) && reduced) {
@@ -958,11 +1030,15 @@ int launch_ragged_strip(const RaggedLaunch &rl, const StripPts<T> &pts, const T 
     // looping over pieces fixes each workgroup's share up front (64-problem
     // benchmark batch: 4.97 vs 5.31 ms)
     const int64_t ub = rl.nunits + pts.M / rl.pmax + rl.nv;
-    const unsigned grid = (unsigned)(ub < (1 << 30) ? ub : (1 << 30));
+    if (ub > INT32_MAX) {
+        set_error("%lld strip pieces are too many for one launch", (long long)ub);
+        return JFA_ERR_TOO_LARGE;
+    }
+    const unsigned grid = (unsigned)ub;
     const T b = (T)beta;
     JFA_DISPATCH_NS(rl.ns, {
         if (phases & kStripSpread)
-            ragged_strip_kernel<T, NS_><<<grid, kStripLanes, 0, stream>>>(
+            ragged_strip_kernel<T, NS_><<<grid, kStripLanes * kRaggedWaves, 0, stream>>>(
                 rl.virt, rl.unit_virt, pts, rl.bin_start, rl.piece_start, rl.npieces,
                 rl.piece_unit, coef, b, kerevalmeth, rl.ptrs, rl.nprob, scratch_all);
         if (phases & kStripMerge) {

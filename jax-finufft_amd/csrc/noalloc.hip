@@ -125,14 +125,13 @@ Buffers carve(Carve &c, const StripGeom &sg, const GridGeom &g, int64_t M, int64
     b.blocksum = c.take<int>(4 * (2 * ((sg.nunits + 255) / 256) + 2));
     b.tile_stride = strip_max_pieces(sg, M) * strip_tile_cells(sg);
     b.tiles = c.take<float>(8 * b.tile_stride);
-    // the sort is done before the tiles are written: its scratch lives there
-    // where it fits
-    const size_t sort_bytes = radix_temp_bytes(m, strip_sort_bits(g.nbins));
-    b.sort_temp = sort_bytes <= (size_t)(8 * b.tile_stride)
-                      ? (void *)b.tiles
-                      : (void *)c.take<unsigned char>(sort_bytes);
     b.fw = c.take<float>(8 * g.nf[0] * g.nf[1]);
-    b.G = c.take<float>(8 * n0 * g.nf[1]);
+    // the FFT's compact buffer is written once the tiles are merged, and fits
+    // them (a tile is larger than the cells that its unit owns)
+    b.G = b.tiles;
+    // the sort is done before the records are packed, and its scratch fits there (8
+    // bytes a point and, per 2048 points, a table of at most 4096)
+    b.sort_temp = b.pack;
     b.tw0 = c.take<float>(8 * g.nf[0]);
     b.tw1 = c.take<float>(8 * g.nf[1]);
     b.coef = c.take<float>(4 * (size_t)nc * g.ns);
@@ -188,7 +187,7 @@ int run_noalloc(jfa_stream_t stream_, float eps, int64_t iflag, int64_t n_tot, i
                   (long long)g.nf[0], (long long)g.nf[1], 2 * g.ns);
         return JFA_ERR_NOT_SUPPORTED;
     }
-    const StripGeom sg = strip_geometry(g, 4096, 8);
+    const StripGeom sg = strip_geometry(g, kStripPiece);
 
     // sizes first, against the array's capacity
     Carve count{nullptr};

@@ -184,18 +184,12 @@ bool jfa::strip_applicable(jfa_plan p) {
     return ((nz * strips * g.nf[1] + 1) << kStripKeyShift) <= (int64_t)UINT32_MAX;
 }
 
-// Strip geometry and bins for the strip spreader, and its buffers.  Units of
-// H rows are sized for about 4096 units (a few waves per SIMD; a 3D grid's
-// slices give many more, so 16 rows there), with H in [ns, nf1 - ns + 1] so
-// that a cell is covered by at most two units per axis.
-// Units a 2D strip geometry aims for: two rounds of the spreading kernel's
-// 5 resident waves per SIMD on 1024 SIMDs.  A wave walks its unit's points in
-// series, so more, shorter units shorten the critical path; the cost is more
-// tile overlap in the merge (2048^2 grid, 1e7 points: 4104 units 0.296 +
-// 0.037 ms spread + merge, 9216 units 0.255 + 0.044 ms).
-static constexpr int64_t kStripTargetUnits = 10240;
-
-jfa::StripGeom jfa::strip_geometry(GridGeom &g, int pmax, int min_h, int rows) {
+// Strip geometry and bins for the strip spreader.  Units are as tall as the
+// spreading kernel's accumulators allow (strip_row_tiles of 16 rows hold H +
+// ns - 1; 9 rows for every ns <= 8): shorter ones only add tile overlap, since a
+// unit's points are spread at the same cost whatever its height.  H stays within
+// [ns, nf1 - ns + 1] so that a cell is covered by at most two units per axis.
+jfa::StripGeom jfa::strip_geometry(GridGeom &g, int pmax, int rows) {
     StripGeom sg{};
     const int ns = g.ns;
     sg.nf0 = g.nf[0];
@@ -204,10 +198,8 @@ jfa::StripGeom jfa::strip_geometry(GridGeom &g, int pmax, int min_h, int rows) {
     sg.nz = g.dim == 3 ? (int)g.nf[2] : 1;
     sg.SW = 64 - ns + 1;
     sg.S = (int)((g.nf[0] + sg.SW - 1) / sg.SW);
-    // 2D: about kStripTargetUnits units (one wave each); 3D: 16-row units
-    int64_t H = sg.nz > 1 ? 16 : (g.nf[1] * sg.S + kStripTargetUnits - 1) / kStripTargetUnits;
-    if (H < min_h) H = min_h;
-    if (rows > 0) H = rows;  // an explicit unit height (gpu_binsizey)
+    const int64_t most = ns <= 8 ? 9 : 33 - ns;
+    int64_t H = rows > 0 ? std::min<int64_t>(rows, most) : most;  // rows: gpu_binsizey
     if (H > g.nf[1] - ns + 1) H = g.nf[1] - ns + 1;
     if (H < ns) H = ns;
     sg.H = (int)H;
@@ -231,8 +223,7 @@ jfa::StripGeom jfa::strip_geometry(GridGeom &g, int pmax, int min_h, int rows) {
 int jfa::setup_strip(jfa_plan p) {
     GridGeom &g = p->geom;
     StripGeom &sg = p->sg;
-    // a single problem fills the GPU with short units
-    sg = strip_geometry(g, p->opts.gpu_maxsubprobsize, 8, p->opts.gpu_binsizey);
+    sg = strip_geometry(g, p->opts.gpu_maxsubprobsize, p->opts.gpu_binsizey);
     // piece table; the tiles are sized by the point count (reserve_strip_scratch)
     free_ptr(reinterpret_cast<void *&>(p->d_piece_start));
     JFA_HIP_CHECK(hipMalloc(&p->d_piece_start, sizeof(int) * (sg.nunits + 1)));
@@ -1221,7 +1212,7 @@ extern "C" int jfa_setpts_info(jfa_plan p, int64_t *info) {
     info[0] = !sorted ? 0 : (strip && p->dim == 3 ? p->M * g.ns : p->M);
     info[1] = g.nbins;
     info[2] = strip ? kStripKeyShift : g.keyshift;
-    info[3] = strip ? 3 : (p->keyed ? g.keyshift : 0);
+    info[3] = strip ? kStripSortLowBit : (p->keyed ? g.keyshift : 0);
     info[4] = p->method;
     info[5] = strip ? 2 : (p->keyed ? 1 : 0);
     for (int d = 0; d < 3; ++d) {
