@@ -82,7 +82,7 @@ constexpr int kStripPiece = 4096;  // default pmax
 // make (sum over units of ceil(count / pmax) <= units + M / pmax).
 inline int64_t strip_tile_cells(const StripGeom &sg) { return (int64_t)(sg.H + sg.ns - 1) * 64; }
 inline int64_t strip_max_pieces(const StripGeom &sg, int64_t M) {
-    return sg.nunits + M / sg.pmax + 1;
+    return std::min<int64_t>(sg.nunits, M) + M / sg.pmax + 1;
 }
 // Units with more than one piece hold more than pmax points each.
 inline int64_t strip_max_heavy(const StripGeom &sg, int64_t M) { return M / (sg.pmax + 1) + 1; }

@@ -488,7 +488,7 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
 // The windows of one axis that reach into window w's first ns - 1 cells from
 // the left: window w - 1, or, for w = 0, the last one or two windows through
 // the periodic wrap (the second when the last window owns fewer than ns - 1
-// cells).  Windows start every `step` cells, span `span` and n of them cover
+// cells), w itself among them where the axis is shorter than a window.  Windows start every `step` cells, span `span` and n of them cover
 // nf cells.  Appends (window, offset of w's cell 0 in its tile) to win / off.
 __device__ __forceinline__ int left_windows(int w, int step, int span, int n, int64_t nf,
                                             int *win, int *off) {
@@ -498,7 +498,7 @@ __device__ __forceinline__ int left_windows(int w, int step, int span, int n, in
         off[c] = step;
         ++c;
     } else {
-        for (int v = n - 1; v >= 1 && v >= n - 2; --v) {
+        for (int v = n - 1; v >= 0 && v >= n - 2; --v) {
             const int o = (int)(nf - (int64_t)v * step);
             if (o < span) {
                 win[c] = v;
@@ -961,7 +961,7 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
     }
     // one workgroup per piece (see launch_ragged_strip); 3D slice grids have
     // tens of thousands of units
-    const int64_t ub = sg.nunits + pts.M / sg.pmax + 1;
+    const int64_t ub = strip_max_pieces(sg, pts.M);
     if (ub > UINT32_MAX / kStripLanes) {  // threads of a launch
         set_error("%lld strip pieces are too many for one launch", (long long)ub);
         return JFA_ERR_TOO_LARGE;

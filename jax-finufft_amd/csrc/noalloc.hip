@@ -124,10 +124,9 @@ Buffers carve(Carve &c, const StripGeom &sg, const GridGeom &g, int64_t M, int64
     b.heavy = c.take<int>(4 * (strip_max_heavy(sg, M) + 1));
     b.blocksum = c.take<int>(4 * (2 * ((sg.nunits + 255) / 256) + 2));
     b.tile_stride = strip_max_pieces(sg, M) * strip_tile_cells(sg);
-    b.tiles = c.take<float>(8 * b.tile_stride);
+    b.tiles = c.take<float>(8 * std::max(b.tile_stride, n0 * g.nf[1]));
     b.fw = c.take<float>(8 * g.nf[0] * g.nf[1]);
-    // the FFT's compact buffer is written once the tiles are merged, and fits
-    // them (a tile is larger than the cells that its unit owns)
+    // the FFT's compact buffer is written once the tiles are merged
     b.G = b.tiles;
     // the sort is done before the records are packed, and its scratch fits there (8
     // bytes a point and, per 2048 points, a table of at most 4096)

@@ -116,7 +116,7 @@ int resolve_method(jfa_plan p) {
     const bool spreads = p->type != 2;
     if (m == JFA_METHOD_STRIP || (m == JFA_METHOD_AUTO && spreads && strip_applicable(p))) {
         if (spreads) {
-            if (!strip_applicable(p)) {
+            if (!strip_applicable(p) || (m == JFA_METHOD_STRIP && p->geom.nf[0] < 64)) {
                 set_error("the strip method needs a 2D or 3D grid of at least 64 x %d (x %d) "
                           "cells", 2 * p->geom.ns, 2 * p->geom.ns);
                 return -1;
@@ -174,10 +174,18 @@ struct DeviceGuard {
 
 // ------------------------------------------------------------------ strips
 
+// Grids of fewer columns than a strip's 64 use part of the tile and are still far
+// faster here than with float atomics in LDS tiles: whole calls of 200,000 points on
+// 24^3 modes 1302 -> 176 us (fp32, 7 digits), 9260 -> 577 (fp64, 9 digits); 300,000
+// on 31^2 319 -> 136 (fp32); 10,000 on 16 x 24 145 -> 122 (fp64, 9 digits).  Their
+// tiles are up to seven times the grid, so only up to kNarrowRows rows (at most 2 GB
+// of tiles in fp32, 4 in fp64 for one transform).
+static constexpr int64_t kNarrowRows = 1 << 20;
 bool jfa::strip_applicable(jfa_plan p) {
     const GridGeom &g = p->geom;
-    if (p->dim < 2 || g.nf[0] < 64 || g.nf[1] < 2 * g.ns) return false;
+    if (p->dim < 2 || g.nf[0] < 2 * g.ns || g.nf[1] < 2 * g.ns) return false;
     if (p->dim == 3 && g.nf[2] < 2 * g.ns) return false;
+    if (g.nf[0] < 64 && g.nf[1] * g.nf[2] > kNarrowRows) return false;
     // (slice, strip, row) bins shifted by the column bits must fit 32-bit sort keys
     const int64_t strips = (g.nf[0] + 64 - g.ns) / (64 - g.ns + 1);
     const int64_t nz = p->dim == 3 ? g.nf[2] : 1;
@@ -254,6 +262,7 @@ static int reserve_strip_scratch(jfa_plan p, int64_t M) {
         (size_t)p->batch * p->strip_scratch_stride * 2 * (p->is_double ? 8 : 4);
     if (bytes > p->strip_scratch_bytes) {
         free_ptr(p->d_strip_scratch);
+        p->strip_scratch_bytes = 0;
         if (hipMalloc(&p->d_strip_scratch, bytes) != hipSuccess) {
             (void)hipGetLastError();
             set_error("could not allocate %zu bytes of strip scratch", bytes);
@@ -675,7 +684,9 @@ int jfa::default_maxsub(jfa_plan p) {
 // (300,007 centre-dense points, 4 transforms, 640 x 512: spreading 168 us in pieces of
 // 4096, 65 us by this rule); evenly filled units stay whole, since every
 // extra piece writes a tile and is summed again (4e6 uniform points on 1024^2
-// in halves: 121 -> 137 us, and 10 us of reduction).
+// in halves: 121 -> 137 us, and 10 us of reduction).  Grids of so few units that they
+// leave the GPU idle are split into 512 pieces, down to 256 points (10,000 fp64 points
+// on 16 x 24 modes, 3 units: 330 -> 123 us a call).
 static void size_chunks(jfa_plan p, int64_t M) {
     if (p->opts.gpu_maxsubprobsize > 0) return;
     auto chunk = [](int64_t v, int64_t most) {
@@ -685,7 +696,9 @@ static void size_chunks(jfa_plan p, int64_t M) {
     p->maxsub = std::max(p->geom.nbins, M / full) < 512 ? chunk(M / 2048, full) : full;
     if (p->method == JFA_METHOD_STRIP) {
         const int64_t Mq = p->dim == 3 ? M * p->geom.ns : M;
-        p->sg.pmax = chunk(std::max(2 * Mq / p->sg.nunits, Mq * p->batch / 4096), kStripPiece);
+        const int64_t all = Mq * p->batch;
+        p->sg.pmax = chunk(std::max(std::min(2 * Mq / p->sg.nunits, all / 512), all / 4096),
+                           kStripPiece);
     }
 }
 

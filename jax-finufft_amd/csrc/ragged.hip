@@ -336,7 +336,7 @@ int check_layout(jfa_ragged r) {
             (int64_t)v.sg.K * v.sg.H < g.nf[1])
             return bad("strip geometry", v.sg.S * v.sg.SW, g.nf[0]);
         // the units' pieces: one per unit at least, one more per pmax points
-        if (strip_max_pieces(v.sg, v.m) < v.sg.nunits + v.m / v.sg.pmax) return bad("piece bound", strip_max_pieces(v.sg, v.m), v.sg.nunits);
+        if (strip_max_pieces(v.sg, v.m) < std::min<int64_t>(v.sg.nunits, v.m) + v.m / v.sg.pmax) return bad("piece bound", strip_max_pieces(v.sg, v.m), v.sg.nunits);
         pieces += strip_max_pieces(v.sg, v.m);
         heavy += strip_max_heavy(v.sg, v.m);
         fw_end = std::max(fw_end, v.fw_off + F);

@@ -31,6 +31,21 @@ def _spread(grid, x, c, eps, prec, method, kerevalmeth, pmax=0):
     return host(out)
 
 
+# fewer columns than a strip: one strip that wraps onto itself, or a second of few
+@pytest.mark.parametrize("columns", [32, 33, 48, 49, 50, 53, 57, 58, 60, 61, 63])
+@pytest.mark.parametrize("prec,eps", [("f32", 1e-2), ("f32", 1e-4), ("f32", 1e-6),
+                                      ("f64", 1e-7), ("f64", 1e-11), ("f64", 1e-15)])
+def test_narrow_grids_match_scatter(prec, eps, columns):
+    rng = np.random.default_rng(58)
+    bar = 64 * (np.finfo(np.float32).eps if prec == "f32" else np.finfo(np.float64).eps) / 2
+    for grid, M in (((32, columns), 33), ((75, columns), 9001), ((33, 34, columns), 2500)):
+        x = uniform_points(rng, len(grid), M, prec)
+        c = cnormal(rng, M, prec)
+        a = _spread(grid, x, c, eps, prec, 0, 1)
+        b = _spread(grid, x, c, eps, prec, 1, 1)
+        assert rel_l2(a, b) <= bar, (grid, M)
+
+
 @pytest.mark.parametrize("prec,eps", WIDTHS)
 @pytest.mark.parametrize("kerevalmeth", [0, 1])
 def test_tiles_match_scatter(prec, eps, kerevalmeth):
