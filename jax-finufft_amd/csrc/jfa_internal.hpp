@@ -372,12 +372,13 @@ template <typename T>
 int launch_t3_prephase(int dim, int64_t M, int ntr, const T *x, const T *y, const T *z,
                        const double *C, const double *D, int iflag, const T *c, T *cp,
                        hipStream_t stream);
-// dec[k] = 1 / prod_d psi_hat(h_d gam_d (s_dk - D_d)) from a quadrature table
-// (wt[q], sn[q]): psi_hat(w) = ns sum_q wt[q] cos(w ns sn[q] / 2).
+// dec[k] = 1 / prod_d psi_hat(h_d gam_d (s_dk - D_d)) from the plan's table: in fp64
+// the quadrature's (wt[q], sn[q]), psi_hat(w) = ns sum_q wt[q] cos(w ns sn[q] / 2); in
+// fp32 the series of kernel_fourier_series over |w| <= range.
 template <typename T>
 int launch_t3_deconv_factors(int dim, int64_t N, const T *s, const T *t, const T *u,
-                             const double *D, const double *hg, int ns, int nq,
-                             const double *quad, T *dec, hipStream_t stream);
+                             const double *D, const double *hg, int ns, double range,
+                             const double *table, T *dec, hipStream_t stream);
 // f[t][k] *= exp(i iflag sum_d s_dk C_d) * dec[k]
 template <typename T>
 int launch_t3_postphase(int dim, int64_t N, int ntr, const T *s, const T *t, const T *u,

@@ -45,6 +45,10 @@ void gauss_legendre(int n, double *x, double *w);
 // returns q.
 constexpr int kMaxFourierNodes = 2 * kMaxNs + 40;
 int kernel_fourier_nodes(int ns, double beta, double *sn, double *wt);
+// The same as a series for |omega| <= range <= 1.02 pi: psi_hat(omega) / ns = sum_j
+// coef[j] T_j(2 (omega / range)^2 - 1) over nt = ns + 20 Chebyshev polynomials;
+// returns nt.
+int kernel_fourier_series(int ns, double beta, double range, double *coef);
 
 // ------------------------------------------------------------ errors
 

@@ -110,6 +110,40 @@ __global__ void __launch_bounds__(256)
     dec[k] = (T)(1.0 / prod);
 }
 
+// The same in fp32, from the Chebyshev series of psi_hat / ns over |w| <= 1 / inv_range:
+// two fp64 operations per term and axis instead of a cosine per node, so that the
+// factors cost little more than reading the targets.  ns = 8, three axes, 2^20
+// targets: 56 cosines an axis 352 us, 28 terms 16 us.  (An fp64 plan keeps the
+// quadrature: the series' last digits are no better, see kernel_fourier_series.)
+template <int DIM>
+__global__ void __launch_bounds__(256)
+    t3_deconv_series_kernel(int64_t N, const float *__restrict__ s, const float *__restrict__ t,
+                            const float *__restrict__ u, V3 D, V3 hg, int ns, int nt,
+                            double inv_range, const double *__restrict__ coef,
+                            float *__restrict__ dec) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= N) return;
+    const float *ss[3] = {s, t, u};
+    double v2[DIM], b1[DIM], b2[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        const double r = hg.v[d] * ((double)ss[d][k] - D.v[d]) * inv_range;
+        v2[d] = 4.0 * r * r - 2.0;  // 2 v
+        b1[d] = b2[d] = 0.0;
+    }
+    for (int j = nt - 1; j > 0; --j)
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            const double b = fma(v2[d], b1[d], coef[j] - b2[d]);
+            b2[d] = b1[d];
+            b1[d] = b;
+        }
+    double prod = 1.0;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) prod *= ns * fma(0.5 * v2[d], b1[d], coef[0] - b2[d]);
+    dec[k] = (float)(1.0 / prod);
+}
+
 template <typename T, int DIM>
 __global__ void __launch_bounds__(256)
     t3_postphase_kernel(int64_t N, int ntr, const T *__restrict__ s, const T *__restrict__ t,
@@ -267,12 +301,19 @@ int launch_t3_prephase(int dim, int64_t M, int ntr, const T *x, const T *y, cons
 
 template <typename T>
 int launch_t3_deconv_factors(int dim, int64_t N, const T *s, const T *t, const T *u,
-                             const double *D, const double *hg, int ns, int nq,
-                             const double *quad, T *dec, hipStream_t stream) {
+                             const double *D, const double *hg, int ns, double range,
+                             const double *table, T *dec, hipStream_t stream) {
     if (N == 0) return JFA_OK;
     unsigned blocks = (unsigned)((N + 255) / 256);
-    JFA_DISPATCH_DIM(dim, t3_deconv_kernel<T, DIM_><<<blocks, 256, 0, stream>>>(
-                              N, s, t, u, v3(D, dim), v3(hg, dim), ns, nq, quad, dec));
+    if constexpr (sizeof(T) == 4) {
+        JFA_DISPATCH_DIM(dim, t3_deconv_series_kernel<DIM_><<<blocks, 256, 0, stream>>>(
+                                  N, s, t, u, v3(D, dim), v3(hg, dim), ns, ns + 20, 1.0 / range,
+                                  table, dec));
+    } else {
+        JFA_DISPATCH_DIM(dim, t3_deconv_kernel<T, DIM_><<<blocks, 256, 0, stream>>>(
+                                  N, s, t, u, v3(D, dim), v3(hg, dim), ns, 2 * ns + 40, table,
+                                  dec));
+    }
     JFA_HIP_CHECK(hipGetLastError());
     return JFA_OK;
 }
@@ -329,7 +370,7 @@ int launch_t3_unsort(int64_t N, int nb, int nbox, const int64_t *start, const in
                                        const double *, const double *, int, const T *, T *,   \
                                        hipStream_t);                                           \
     template int launch_t3_deconv_factors<T>(int, int64_t, const T *, const T *, const T *,    \
-                                             const double *, const double *, int, int,         \
+                                             const double *, const double *, int, double,        \
                                              const double *, T *, hipStream_t);                \
     template int launch_t3_postphase<T>(int, int64_t, int, const T *, const T *, const T *,    \
                                         const double *, int, const T *, T *, hipStream_t);

@@ -183,6 +183,31 @@ int kernel_fourier_nodes(int ns, double beta, double *sn, double *wt) {
     return q;
 }
 
+// Interpolation at ns + 24 Chebyshev points.  cos(a s) is entire, and as a series in
+// even Chebyshev polynomials over |a| <= A = range ns / 2 its coefficients are
+// 2 J_2j(A s): at 2j = 2 ns + 40 below 1e-17 for every ns <= 16 (A <= 25.6).  Against
+// the quadrature in extended precision the series is off by at most 3.7e-15 of
+// psi_hat at sigma = 2 and 2.9e-13 at sigma = 1.25 (the quadrature in doubles: 9.7e-16
+// and 2.1e-13).
+int kernel_fourier_series(int ns, double beta, double range, double *coef) {
+    const int K = ns + 24, nt = ns + 20;
+    std::vector<double> sn(kMaxFourierNodes), wt(kMaxFourierNodes), cs(4 * K), f(K);
+    const int q = kernel_fourier_nodes(ns, beta, sn.data(), wt.data());
+    for (int m = 0; m < 4 * K; ++m) cs[m] = std::cos(m * M_PI / (2 * K));
+    for (int i = 0; i < K; ++i) {
+        // v = cos((i + 1/2) pi / K), sqrt((v + 1) / 2) = cos((i + 1/2) pi / 2K)
+        const double a = 0.5 * ns * range * std::cos((i + 0.5) * M_PI / (2 * K));
+        f[i] = 0.0;
+        for (int p = 0; p < q; ++p) f[i] += wt[p] * std::cos(a * sn[p]);
+    }
+    for (int j = 0; j < nt; ++j) {
+        double c = 0.0;
+        for (int i = 0; i < K; ++i) c += f[i] * cs[j * (2 * i + 1) % (4 * K)];
+        coef[j] = c * (j ? 2.0 : 1.0) / K;
+    }
+    return nt;
+}
+
 void kernel_fourier_at(int ns, double beta, const double *omega, int64_t n, double *out) {
     std::vector<double> sn(kMaxFourierNodes), wt(kMaxFourierNodes);
     const int q = kernel_fourier_nodes(ns, beta, sn.data(), wt.data());

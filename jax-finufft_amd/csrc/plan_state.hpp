@@ -91,7 +91,7 @@ struct jfa_plan_s {
     void *d_t3_deconv = nullptr;  // per-target 1 / prod psi_hat (real)
     int64_t cap_t3_deconv = 0;
     double *d_minmax = nullptr;   // scratch for extents (6 x [min, max]) and their partials
-    void *d_quad = nullptr;       // quadrature table for psi_hat at arbitrary omega
+    void *d_quad = nullptr;       // quadrature (fp64) or series (fp32) of psi_hat at arbitrary omega
     // type 3 over boxes of targets, when one pair of grids would exceed the
     // cell limit or the memory budget: k[d] boxes per axis of width
     // t3_box_w[d] from t3_box_lo[d]; targets in box order

@@ -62,25 +62,30 @@ void type3_grid(double X, double S, double sigma, int ns, int64_t *nf, double *h
     *gam = (double)n / (2.0 * sigma * Ss);
 }
 
+// Every target's frequency is at most h gam S = pi / sigma radians per cell (see
+// type3_grid; boxes of targets overlap by rounding only).
+double fourier_range(jfa_plan p) { return 1.02 * M_PI / p->opts.upsampfac; }
+
 }  // namespace
 
 int jfa::type3_init(jfa_plan p) {
     p->geom.dim = p->dim;
     p->geom.ns = p->kp.ns;
-    // Horner table (the spread kernel) and the quadrature table for psi_hat
+    // Horner table (the spread kernel) and the table for psi_hat
     int rc = upload_kernel_tables(p, nullptr);
     if (rc) return rc;
     const int ns = p->kp.ns;
-    const int nq = 2 * ns + 40;
-    std::vector<double> gx(nq), gw(nq), quad(2 * nq);
-    gauss_legendre(nq, gx.data(), gw.data());
-    for (int q = 0; q < nq; ++q) {
-        double th = 0.25 * M_PI * (gx[q] + 1.0);
-        quad[q] = 0.25 * M_PI * gw[q] * std::cos(th) * std::exp(p->kp.beta * (std::cos(th) - 1.0));
-        quad[nq + q] = std::sin(th);
+    std::vector<double> table(2 * kMaxFourierNodes);
+    int n;
+    if (p->is_double) {
+        n = kernel_fourier_nodes(ns, p->kp.beta, table.data() + kMaxFourierNodes, table.data());
+        std::copy_n(table.begin() + kMaxFourierNodes, n, table.begin() + n);
+        n *= 2;
+    } else {
+        n = kernel_fourier_series(ns, p->kp.beta, fourier_range(p), table.data());
     }
-    JFA_HIP_CHECK(hipMalloc(&p->d_quad, sizeof(double) * 2 * nq));
-    JFA_HIP_CHECK(hipMemcpy(p->d_quad, quad.data(), sizeof(double) * 2 * nq, hipMemcpyHostToDevice));
+    JFA_HIP_CHECK(hipMalloc(&p->d_quad, sizeof(double) * n));
+    JFA_HIP_CHECK(hipMemcpy(p->d_quad, table.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     // [min, max] of up to six arrays, then the partials of one pass
     JFA_HIP_CHECK(hipMalloc(&p->d_minmax, sizeof(double) * (12 + 2 * 1024)));
     return JFA_OK;
@@ -350,7 +355,7 @@ static int type3_setpts_t(jfa_plan p, int64_t M, const T *const xs[3], int64_t N
         rc = setpts_12(p->inner, N, ss[0], ss[1], ss[2]);
         if (rc) return rc;
         return launch_t3_deconv_factors<T>(dim, N, ss[0], ss[1], ss[2], p->t3_D, hg, ns,
-                                           2 * ns + 40, (const double *)p->d_quad,
+                                           fourier_range(p), (const double *)p->d_quad,
                                            (T *)p->d_t3_deconv, p->stream);
     }
     // target boxes: box order, box sizes on the host, per-box deconvolution
@@ -400,8 +405,8 @@ static int type3_setpts_t(jfa_plan p, int64_t M, const T *const xs[3], int64_t N
         box_centre(p, b, Db);
         const T *sb[3] = {nullptr, nullptr, nullptr};
         for (int d = 0; d < dim; ++d) sb[d] = sorted + (int64_t)d * N + s0;
-        rc = launch_t3_deconv_factors<T>(dim, nb, sb[0], sb[1], sb[2], Db, hg, ns, 2 * ns + 40,
-                                         (const double *)p->d_quad,
+        rc = launch_t3_deconv_factors<T>(dim, nb, sb[0], sb[1], sb[2], Db, hg, ns,
+                                         fourier_range(p), (const double *)p->d_quad,
                                          (T *)p->d_t3_deconv + s0, p->stream);
         if (rc) return rc;
     }
