@@ -222,10 +222,10 @@ __device__ __forceinline__ PieceRange piece_range(const StripGeom &sg,
 // another to per-lane windows of the tile (10.4 VALU instructions and 9.6 LDS cycles
 // per point) took 268; a unit's points now need no order within a row, which makes
 // the sort's keys 3 bits shorter.  The walk was a chain of LDS reads and adds, so
-// smaller and wider problems gain more: 1e6 fp64 points on 1024^2 at ns = 11 275 ->
-// 185 us, 300,007 points x 3 transforms on 501 x 333 at ns = 6 65 -> 46, 100,000
-// points on 256^2 29 -> 11; 1e6 points and as many targets of a 3D type 3 at ns = 8
-// 507 -> 314.
+// smaller and wider problems gain more: 1e6 fp64 points on 1024^2 cells at ns = 11
+// 275 -> 185 us, 300,007 centre-dense points x 4 transforms on 301 x 255 modes at
+// ns = 6 65 -> 46, 4000 points on 48 x 40 29 -> 11; 2^20 sources of a 3D type 3 at
+// ns = 8 507 -> 314.
 //
 // W waves share a piece: each spreads a run of its points into accumulators of its
 // own, which are added through LDS in wave order at the end.
@@ -969,8 +969,9 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
     const unsigned grid = (unsigned)ub;
     // Waves per piece: four where an even unit has two batches of points or more
     // (shorter waves level the last round, and few units still fill the GPU: 1e7
-    // points on 2048^2 263 us, one wave 276; 1e6 on 512^2 110, one wave 145; 300,007
-    // x 3 on 501 x 333 46, one wave 76); one in sparser units and pieces, where most
+    // points on 2048^2 cells 263 us, one wave 276; 4e6 on 1024^2 110, one wave 145;
+    // 300,007 centre-dense points x 4 transforms on 301 x 255 modes 46, one wave 76);
+    // one in sparser units and pieces, where most
     // of the four would find no points.
     constexpr int kPieceWaves = 4;
     const int waves = std::min<int64_t>(pts.M / sg.nunits, sg.pmax) >= 2 * kStripLanes &&

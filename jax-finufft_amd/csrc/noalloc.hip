@@ -5,7 +5,7 @@
 //
 // Every buffer the transform needs beyond the caller's inputs and output
 // lives in one file-scope device array, `scratch`, of kNoallocBytes per GPU:
-// the sort keys and their rocPRIM temp, the strip bins and piece tables, the
+// the sort keys and the sort's scratch, the strip bins and piece tables, the
 // spreading records and tiles, the fine grid, the compact pruned-FFT buffer,
 // the FFT twiddles and the kernel tables.  Its address on the current device
 // is looked up once per device with hipGetSymbolAddress and kept; kernels are
