@@ -681,8 +681,8 @@ int jfa::default_maxsub(jfa_plan p) {
 // Strip pieces: a wave walks its piece in series, so one crowded unit in full
 // pieces can outlast the rest of the launch.  Units are split above twice the
 // mean unit, and above a wave slot's share of the points of all nb transforms
-// (300,007 centre-dense points, 4 transforms, 640 x 512: spreading 168 us in pieces of
-// 4096, 65 us by this rule); evenly filled units stay whole, since every
+// (300,007 centre-dense points, 4 transforms, 640 x 512 cells: spreading 168 us in
+// pieces of 4096, 65 us by this rule, 46 on matrix instructions); evenly filled units stay whole, since every
 // extra piece writes a tile and is summed again (4e6 uniform points on 1024^2
 // in halves: 121 -> 137 us, and 10 us of reduction).  Grids of so few units that they
 // leave the GPU idle are split into 512 pieces, down to 256 points (10,000 fp64 points
