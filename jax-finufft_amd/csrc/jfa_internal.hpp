@@ -164,11 +164,16 @@ struct RaggedLaunch {
     int *piece_unit;           // global unit of every piece
     int *heavy;                // [count, units with more than one piece ...]
     int64_t max_heavy;         // most such units
+    int64_t max_pieces;        // most pieces, over every virtual problem
     int reduce_chunks;         // 256-cell chunks of the largest tile
     int *blocksum;             // 2 * ceil(nunits / 256) + 1 ints of piece-scan scratch
     int nprob, nv, ns, pmax, keyshift;
     int64_t mtot, nbins, nunits, mode_blocks;
 };
+// Workgroups of the spreading launch, one per piece.  Every transform of a problem
+// has its own pieces, so the points of a problem with T transforms count T times
+// (mtot counts them once).
+inline int64_t ragged_strip_blocks(const RaggedLaunch &rl) { return rl.max_pieces; }
 
 // Points after setpts, in bin-sorted order: original index, first tap
 // (wrapped into [0, nf)) and the Horner variable t = 2*frac - 1 per dim.

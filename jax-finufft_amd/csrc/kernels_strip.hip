@@ -1026,12 +1026,12 @@ int launch_ragged_strip(const RaggedLaunch &rl, const StripPts<T> &pts, const T 
                                                            rl.heavy);
         JFA_HIP_CHECK(hipGetLastError());
     }
-    // one workgroup per piece: piece costs differ by problem density, and the
-    // hardware dispatcher balances them as waves finish, where a capped grid
+    // one workgroup per piece (the kernel does not loop): piece costs differ by
+    // problem density, and the hardware dispatcher balances them as waves finish, where a capped grid
     // looping over pieces fixes each workgroup's share up front (64-problem
     // benchmark batch: 4.97 vs 5.31 ms)
-    const int64_t ub = rl.nunits + pts.M / rl.pmax + rl.nv;
-    if (ub > INT32_MAX) {
+    const int64_t ub = ragged_strip_blocks(rl);
+    if (ub > UINT32_MAX / (kStripLanes * kRaggedWaves)) {  // threads of a launch
         set_error("%lld strip pieces are too many for one launch", (long long)ub);
         return JFA_ERR_TOO_LARGE;
     }

@@ -274,6 +274,7 @@ int layout(jfa_ragged r) {
     rl.nbins = bins;
     rl.nunits = r->vunit_off.back();
     rl.mode_blocks = r->mode_blk.back();
+    rl.max_pieces = r->max_pieces;
     return JFA_OK;
 }
 
@@ -343,6 +344,7 @@ int check_layout(jfa_ragged r) {
         g_end = std::max(g_end, v.g_off + v.n0 * g.nf[1]);
         tile_end = std::max(tile_end, v.tile_off + tiles);
     }
+    if (ragged_strip_blocks(r->rl) < pieces) return bad("spreading workgroups", ragged_strip_blocks(r->rl), pieces);
     if (pieces != r->max_pieces || heavy != r->max_heavy) return bad("piece totals", pieces, r->max_pieces);
     if (fw_end != r->fw_cells || g_end != r->g_cells || tile_end != r->tile_cells) return bad("buffer totals", fw_end, r->fw_cells);
     if (r->rl.mode_blocks != r->mode_blk.back()) return bad("mode block total", r->rl.mode_blocks, r->mode_blk.back());

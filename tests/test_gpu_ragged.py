@@ -118,6 +118,24 @@ def test_ragged_heavy_units_and_output_reuse():
     assert rel_l2(host(out[1]), oracle.type1([x2, y2], c2, shapes[1], 1)) <= 1e-6
 
 
+@pytest.mark.parametrize("T", [3, 8])
+@pytest.mark.parametrize("pmax", [0, 256])
+def test_ragged_many_pieces_a_unit_and_transforms(T, pmax):
+    # small grids, units of many full pieces, several transforms: every
+    # transform's pieces are spread, the last one's too
+    probs = _problems(35, "f32", [((64, 64), 400_000, T, "uniform"),
+                                  ((100, 72), 150_000, T - 2, "clustered")])
+    xs, ys, cs = ([dev(p[k]) for p in probs] for k in (1, 2, 3))
+    plan = RaggedPlan([p[0] for p in probs], [p[1].size for p in probs], [T, T - 2], eps=1e-6,
+                      graph=False, pmax=pmax)
+    got = plan.run(xs, ys, cs)
+    for i, (shape, x, y, c) in enumerate(probs):
+        g = host(got[i]).reshape((-1,) + shape)
+        single = host(nufft1(shape, cs[i], xs[i], ys[i], eps=1e-6)).reshape(g.shape)
+        for t in range(g.shape[0]):
+            assert rel_l2(g[t], single[t]) < TOL_SAME["f32"], (i, t)
+
+
 def test_ragged_rejects_mismatched_inputs():
     plan = RaggedPlan([(64, 64)], [100], [1], eps=1e-6, graph=False)
     x = torch.zeros(100, device="cuda")

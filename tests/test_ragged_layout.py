@@ -76,6 +76,21 @@ def test_edge_batches(L, case):
     assert info[0] == sum(Ms) and info[3] == sum(Ts)
 
 
+@pytest.mark.parametrize("case", [
+    # many full pieces a unit and several transforms: one workgroup per piece
+    # of every transform
+    ([(64, 64)], [3], [2_000_000]),
+    ([(64, 64)], [8], [2_000_000]),
+    ([(128, 128), (33, 40)], [4, 1], [1_000_000, 0]),
+    ([(64, 64), (100, 80)], [5, 2], [100_000, 60_000]),
+])
+@pytest.mark.parametrize("pmax", [0, 256])
+def test_workgroups_cover_every_piece(L, case, pmax):
+    Ns, Ts, Ms = case
+    rc, info = _check(L, Ns, Ts, Ms, gpu_maxsubprobsize=pmax)
+    assert rc == 0, _native.last_error()
+
+
 @pytest.mark.parametrize("seed", range(12))
 def test_random_batches(L, seed):
     rng = np.random.default_rng(100 + seed)
