@@ -671,9 +671,11 @@ int jfa::default_maxsub(jfa_plan p) {
 
 // Subproblem and piece sizes for M points, unless the caller chose one.
 //
-// LDS subproblems: the full size (default_maxsub) once that many bins or chunks, of
-// all transforms of a batch, fill the GPU; with under 512 of them, M nb / 2048 points,
-// never below the 256 lanes of a workgroup (30,011 fp64 points on 2048 cells, 1D interpolation:
+// LDS subproblems: the full size (default_maxsub) once that many bins or chunks
+// fill the GPU; with under 512 of them, M nb / 2048 points (nb transforms read the
+// points; 2D type 2, 64^2 modes, 300,000 points, 8 transforms: 256 points 59 us in
+// fp32 and 155 in fp64, 1171 points 47 and 127), never below the 256 lanes of a
+// workgroup (30,011 fp64 points on 2048 cells, 1D interpolation:
 // 8 workgroups 187 us, 118 workgroups 7 us).  Splitting where there are enough
 // only reloads tiles: 1e7 points in 1024 bins of 64 x 64, halves instead of
 // whole bins, 0.265 -> 0.367 ms.
@@ -693,10 +695,7 @@ static void size_chunks(jfa_plan p, int64_t M) {
         return (int)std::min(most, std::max<int64_t>(256, (v + 63) / 64 * 64));
     };
     const int full = default_maxsub(p);
-    const int64_t slots = p->type == 2 ? 1024 : 512, all_M = M * p->batch;
-    p->maxsub = std::max(p->geom.nbins, M / full) * p->batch < slots
-                    ? chunk(all_M / (p->type == 2 ? 1024 : 2048), full)
-                    : full;
+    p->maxsub = std::max(p->geom.nbins, M / full) < 512 ? chunk(M * p->batch / 2048, full) : full;
     if (p->method == JFA_METHOD_STRIP) {
         const int64_t Mq = p->dim == 3 ? M * p->geom.ns : M;
         const int64_t all = Mq * p->batch;
