@@ -133,24 +133,45 @@ struct StripLds {
     T kx[StripShape<NS>::kValues];
 };
 
-// The ns weights of a point along one axis to LDS.  Doubles a few taps at a time:
-// all chains at once need more registers than the accumulators leave.
+// The ns weights of a point along one axis to LDS, as eval_kernel computes them.  Wide
+// double kernels two taps at a time, in a loop: the accumulators leave no registers for
+// every tap at once.
 template <typename T, int NS, typename Coef>
 __device__ __forceinline__ void stage_weights(Coef coef, T beta, int horner, T t, T *out) {
-    if (sizeof(T) == 8 && NS > 8 && horner) {
-        constexpr int NC = horner_nc(NS), NE = (NC + 1) / 2, NO = NC / 2;  // as in eval_kernel
-        const T s = t * t;
-        unroll<(NS + 1) / 2>([&](auto ic) {
-            constexpr int i = decltype(ic)::value;
-            T e = coef[2 * (NE - 1) * NS + i], o = coef[(2 * NO - 1) * NS + i];
+    if constexpr (sizeof(T) == 8 && NS > 8) {
+        if (horner) {
+            constexpr int NC = horner_nc(NS), NE = (NC + 1) / 2, NO = NC / 2, half = (NS + 1) / 2;
+            const T s = t * t;
+#pragma unroll 1
+            for (int i = 0; i < half; i += 2) {
+                const Coef c = coef + i;
+                T e0 = c[2 * (NE - 1) * NS], e1 = c[2 * (NE - 1) * NS + 1];
+                T o0 = c[(2 * NO - 1) * NS], o1 = c[(2 * NO - 1) * NS + 1];
 #pragma unroll
-            for (int k = NE - 2; k >= 0; --k) e = fma(e, s, coef[2 * k * NS + i]);
+                for (int k = NE - 2; k >= 0; --k) {
+                    e0 = fma(e0, s, c[2 * k * NS]);
+                    e1 = fma(e1, s, c[2 * k * NS + 1]);
+                }
 #pragma unroll
-            for (int k = NO - 2; k >= 0; --k) o = fma(o, s, coef[(2 * k + 1) * NS + i]);
-            out[i] = fma(t, o, e);
-            if constexpr (NS - 1 - i != i) out[NS - 1 - i] = fma(-t, o, e);
-            if constexpr (i % 2 == 1) __builtin_amdgcn_sched_barrier(0);
-        });
+                for (int k = NO - 2; k >= 0; --k) {
+                    o0 = fma(o0, s, c[(2 * k + 1) * NS]);
+                    o1 = fma(o1, s, c[(2 * k + 1) * NS + 1]);
+                }
+                out[NS - 1 - i] = fma(-t, o0, e0);
+                out[i] = fma(t, o0, e0);
+                if (half % 2 == 0 || i + 1 < half) {
+                    out[NS - 2 - i] = fma(-t, o1, e1);
+                    out[i + 1] = fma(t, o1, e1);
+                }
+            }
+        } else {
+#pragma unroll 1
+            for (int i = 0; i < NS; ++i) {
+                const T z = (T(-0.5 * NS) + T(i) + T(0.5) * (t + T(1))) * (T(2) / T(NS));
+                const T a = T(1) - z * z;
+                out[i] = a < T(0) ? T(0) : exp(beta * (sqrt(a) - T(1)));
+            }
+        }
         return;
     }
     T k[NS];
