@@ -988,17 +988,20 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
         return JFA_ERR_TOO_LARGE;
     }
     const unsigned grid = (unsigned)ub;
-    // Waves per piece: four where an even unit has two batches of points or more
-    // (shorter waves level the last round, and few units still fill the GPU: 1e7
-    // points on 2048^2 cells 263 us, one wave 276; 4e6 on 1024^2 110, one wave 145;
-    // 300,007 centre-dense points x 4 transforms on 301 x 255 modes 46, one wave 76);
-    // one in sparser units and pieces, where most
-    // of the four would find no points.
+    // Waves per piece: four fill the GPU where units are few, and level the last round
+    // where they hold many points; with many units of fewer points one wave does less
+    // work (a tile to sum instead of four).  Even units' points, and where the line lies:
+    // w = 8 in fp32, one wave / four: 737 units of 271 points 21 / 16 us, 2052 of 292 30 /
+    // 32, 2052 of 585 51 / 46, 8208 of 487 111 / 128, 37,120 of 216 217 / 350, 8208 of
+    // 1219 276 / 263.  Narrow fp64 kernels hold half as many waves and are bound by their
+    // products sooner (737 of 271 28 / 33, 2052 of 585 82 / 88, of 1170 153 / 137).
+    const bool narrow64 = sizeof(T) == 8 && sg.ns <= 8;
+    const int64_t even = std::min<int64_t>(pts.M / sg.nunits, sg.pmax);
+    const int64_t line = std::min<int64_t>(
+        std::max<int64_t>((int64_t)sg.nunits * ntr, 512) / (narrow64 ? 2 : 4), narrow64 ? 2048 : 1024);
     constexpr int kPieceWaves = 4;
-    const int waves = std::min<int64_t>(pts.M / sg.nunits, sg.pmax) >= 2 * kStripLanes &&
-                              ub <= UINT32_MAX / (kStripLanes * kPieceWaves)
-                          ? kPieceWaves
-                          : 1;
+    const int waves =
+        even >= line && ub <= UINT32_MAX / (kStripLanes * kPieceWaves) ? kPieceWaves : 1;
     const T b = (T)beta;
     JFA_DISPATCH_NS(sg.ns, {
         if (phases & kStripSpread) {
