@@ -82,7 +82,8 @@ typedef struct {
     int gpu_maxbatchsize;  /* transforms per spread/FFT batch; 0 = all */
     int debug;             /* 1: print per-stage timings to stderr */
     int gpu_binsizex, gpu_binsizey, gpu_binsizez; /* LDS-tile bins; for the strip
-                              method gpu_binsizey is the unit height in rows;
+                              method gpu_binsizey asks for the unit height in rows,
+                              of which a unit has w to 33 - w;
                               0 = default (or the autotuner's choice) */
     int gpu_maxsubprobsize;  /* points per LDS subproblem / strip piece; 0 = default */
     int gpu_spreadinterponly; /* 1: execute spreads/interpolates only; the mode

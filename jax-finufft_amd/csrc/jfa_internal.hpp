@@ -87,12 +87,21 @@ inline int64_t strip_max_pieces(const StripGeom &sg, int64_t M) {
 // Units with more than one piece hold more than pmax points each.
 inline int64_t strip_max_heavy(const StripGeom &sg, int64_t M) { return M / (sg.pmax + 1) + 1; }
 
-// Rows of the spreading kernel's accumulators, in tiles of 16: a unit's H +
-// ns - 1 rows fit them.
-constexpr int strip_row_tiles(int ns) { return ns <= 8 ? 1 : 2; }
-// Strip geometry for a grid g (nf and ns set), with units of H rows; also sets
-// g's bins to (strip, row), rows fastest.  rows > 0 asks for lower units.
-StripGeom strip_geometry(GridGeom &g, int pmax, int rows = 0);
+// Most rows of a unit that the spreading kernel's accumulators hold: short units, and
+// the tall ones of sparse grids (the same for ns > 8).
+constexpr int strip_short_rows(int ns) { return ns <= 8 ? 9 : 33 - ns; }
+constexpr int strip_tall_rows(int ns) { return 33 - ns; }
+// Strips of a grid g (nf and ns set) in short units; also sets g's bins to (strip, row),
+// rows fastest, which do not depend on the units.
+StripGeom strip_geometry(GridGeom &g, int pmax);
+// Sets the height of the units, as near `rows` as they may have.
+void strip_set_rows(StripGeom &sg, int64_t rows);
+// Whether tall units suit that many points (slice points in 3D) in all of so many short
+// units, over every transform.
+bool strip_tall(double points, double units);
+// Sets the height that suits M points of nb transforms; rows > 0 asks for one
+// (gpu_binsizey).
+void strip_units(StripGeom &sg, int64_t M, int nb, int rows);
 int ensure_rocfft();
 
 // Batched 1D FFTs in LDS (fft_lds.hip), for rows of length n = 2^a 3^b 5^c <=
@@ -165,6 +174,7 @@ struct RaggedLaunch {
     int *heavy;                // [count, units with more than one piece ...]
     int64_t max_heavy;         // most such units
     int64_t max_pieces;        // most pieces, over every virtual problem
+    bool tall;                 // units of more than strip_short_rows rows
     int reduce_chunks;         // 256-cell chunks of the largest tile
     int *blocksum;             // 2 * ceil(nunits / 256) + 1 ints of piece-scan scratch
     int nprob, nv, ns, pmax, keyshift;

@@ -94,11 +94,12 @@ struct Mfma<double> {
     static __device__ __forceinline__ int row(int r, int g) { return 4 * r + g; }
 };
 
-// Shape of a unit's tile in MFMA terms (see strip_piece).
-template <int NS>
+// Shape of a unit's tile in MFMA terms (see strip_piece).  TALL: units of more than
+// strip_short_rows rows, ns <= 8 (wider kernels' shape is always the tall one).
+template <int NS, bool TALL>
 struct StripShape {
-    static constexpr bool kNarrow = NS <= 8;
-    static constexpr int kRowTiles = strip_row_tiles(NS);  // of 16 rows
+    static constexpr bool kNarrow = NS <= 8 && !TALL;
+    static constexpr int kRowTiles = kNarrow ? 1 : 2;  // of 16 rows
     // narrow: frames start every 8 columns, so one 16-column frame holds a
     // point's taps; wide: every 16 columns, a point reaches into the next frame
     static constexpr int kFrames = kNarrow ? 8 : 4;
@@ -126,11 +127,11 @@ struct alignas(16) StripSlot {
 
 // LDS staging of one wave: the weights by point of the batch, the points by slot.
 // (ns <= 8 in fp32: 10,232 bytes, so that 16 waves share a CU's 160 KiB.)
-template <typename T, int NS, int NT = 1>
+template <typename T, int NS, int NT, bool TALL>
 struct StripLds {
-    StripSlot<T, NT> slot[StripShape<NS>::kSlots];
-    T ky[StripShape<NS>::kValues];
-    T kx[StripShape<NS>::kValues];
+    StripSlot<T, NT> slot[StripShape<NS, TALL>::kSlots];
+    T ky[StripShape<NS, TALL>::kValues];
+    T kx[StripShape<NS, TALL>::kValues];
 };
 
 // The ns weights of a point along one axis to LDS, as eval_kernel computes them.  Wide
@@ -229,8 +230,8 @@ __device__ __forceinline__ PieceRange piece_range(const StripGeom &sg,
 // The accumulators hold the unit's tile: rows r0 .. r0 + 16 kRowTiles - 1 by
 // frames of 16 columns.  ns <= 8: eight frames 8 columns apart, one row tile, so a
 // point adds to exactly one frame: one MFMA each for the real and imaginary parts
-// of four points (half the columns are zeros).  ns > 8: four frames, two row
-// tiles; a point adds to its frame and the next, and to both row tiles where its
+// of four points (half the columns are zeros).  ns > 8, and tall units of ns <= 8
+// (strip_tall): four frames, two row tiles; a point adds to its frame and the next, and to both row tiles where its
 // rows straddle them (batches are in row order, so a row tile no point of the
 // batch touches is skipped).  Each MFMA's four points must share a frame: the
 // points of a batch are ranked by frame (one ballot per bit of the frame) and
@@ -250,19 +251,19 @@ __device__ __forceinline__ PieceRange piece_range(const StripGeom &sg,
 //
 // W waves share a piece: each spreads a run of its points into accumulators of its
 // own, which are added through LDS in wave order at the end.
-template <typename T, int NS, int NT, int W>
+template <typename T, int NS, int NT, int W, bool TALL>
 __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<T> &pts,
                                             const int *__restrict__ bin_start, int u, int sub,
                                             const T *__restrict__ coef, T beta, int horner,
                                             T *__restrict__ tile, int64_t tile_tstride,
-                                            StripLds<T, NS, NT> *lds_all) {
-    using Sh = StripShape<NS>;
+                                            StripLds<T, NS, NT, TALL> *lds_all) {
+    using Sh = StripShape<NS, TALL>;
     using M = Mfma<T>;
     using Acc = typename M::Acc;
     constexpr int RT = Sh::kRowTiles, NF = Sh::kFrames, S = Sh::kStride;
     const int lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
     const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
-    StripLds<T, NS, NT> &lds = lds_all[wave];
+    StripLds<T, NS, NT, TALL> &lds = lds_all[wave];
     const PieceRange pr = piece_range(sg, bin_start, u, sub);
     const int r0 = pr.r0;
     // this wave's points: whole batches, as even as they come
@@ -479,7 +480,7 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
     } else {
         // eight values of every lane at a time through the staging areas; wave w
         // adds up values w, w + W, ...
-        static_assert(sizeof(StripLds<T, NS, NT>) >= 8 * kStripLanes * sizeof(Pair<T>), "");
+        static_assert(sizeof(StripLds<T, NS, NT, TALL>) >= 8 * kStripLanes * sizeof(Pair<T>), "");
         __syncthreads();
         unroll<NT * RT * 2>([&](auto cc) {
             constexpr int e0 = 8 * decltype(cc)::value;
@@ -651,22 +652,22 @@ __device__ __forceinline__ void piece_scan(int n, PiecesOf pieces, int *piece_st
 template <typename T, int NT>
 constexpr int strip_waves() { return sizeof(T) * NT == 4 ? 4 : sizeof(T) * NT == 8 ? 2 : 1; }
 
-template <typename T, int NS, int W>
+template <typename T, int NS, int W, bool TALL>
 __global__ void __launch_bounds__(kStripLanes *W, (strip_waves<T, 1>()))
     spread_strip_kernel(StripGeom sg, StripPts<T> pts, const int *__restrict__ bin_start,
                         const int *__restrict__ piece_start, const int *__restrict__ npieces,
                         const int *__restrict__ piece_unit, const T *__restrict__ coef, T beta,
                         int horner, int64_t pack_stride, T *__restrict__ scratch,
                         int64_t scratch_stride) {
-    __shared__ StripLds<T, NS> lds[W];
+    __shared__ StripLds<T, NS, 1, TALL> lds[W];
     pts.pack += 4 * pack_stride * blockIdx.y;
     scratch += 2 * scratch_stride * blockIdx.y;
     const int64_t tile_cells = (int64_t)(sg.H + NS - 1) * kStripLanes;
     const int piece = blockIdx.x;  // one workgroup per piece
     if (piece >= *npieces) return;
     const int u = piece_unit[piece];
-    strip_piece<T, NS, 1, W>(sg, pts, bin_start, u, piece - piece_start[u], coef, beta, horner,
-                             scratch + 2 * piece * tile_cells, 0, lds);
+    strip_piece<T, NS, 1, W, TALL>(sg, pts, bin_start, u, piece - piece_start[u], coef, beta,
+                                   horner, scratch + 2 * piece * tile_cells, 0, lds);
 }
 
 // pack[t][j] = (c[t][j], rec[j])
@@ -878,7 +879,7 @@ __global__ void __launch_bounds__(256)
 // Waves per piece.  Problems of all densities fill the GPU together: 64 problems of
 // up to 2e6 points, 1 to 8 transforms: the batch takes 4.70 ms, with four 6.03.
 constexpr int kRaggedWaves = 1;
-template <typename T, int NS>
+template <typename T, int NS, bool TALL>
 __global__ void __launch_bounds__(kStripLanes *kRaggedWaves, (strip_waves<T, 2>()))
     ragged_strip_kernel(const RaggedVirt *__restrict__ virt, const int *__restrict__ unit_virt,
                         StripPts<T> pts, const int *__restrict__ bin_start,
@@ -887,7 +888,7 @@ __global__ void __launch_bounds__(kStripLanes *kRaggedWaves, (strip_waves<T, 2>(
                         const T *__restrict__ coef, T beta, int horner,
                         const void *const *__restrict__ ptrs, int nprob,
                         T *__restrict__ scratch_all) {
-    __shared__ StripLds<T, NS, 2> lds[kRaggedWaves];
+    __shared__ StripLds<T, NS, 2, TALL> lds[kRaggedWaves];
     const int piece = blockIdx.x;  // one workgroup per piece
     if (piece >= *npieces) return;
     const int gu = piece_unit[piece];
@@ -903,12 +904,13 @@ __global__ void __launch_bounds__(kStripLanes *kRaggedWaves, (strip_waves<T, 2>(
     const int64_t tile_cells = (int64_t)(d.sg.H + NS - 1) * kStripLanes;
     T *tile = scratch_all + 2 * (d.tile_off + (piece - piece_start[d.unit_off]) * tile_cells);
     if (d.nt > 1)
-        strip_piece<T, NS, 2, kRaggedWaves>(d.sg, vp, bin_start + d.bin_off, gu - d.unit_off, sub,
-                                            coef, beta, horner, tile, 2 * d.tile_next, lds);
+        strip_piece<T, NS, 2, kRaggedWaves, TALL>(d.sg, vp, bin_start + d.bin_off,
+                                                   gu - d.unit_off, sub, coef, beta, horner, tile,
+                                                   2 * d.tile_next, lds);
     else
-        strip_piece<T, NS, 1, kRaggedWaves>(d.sg, vp, bin_start + d.bin_off, gu - d.unit_off, sub,
-                                            coef, beta, horner, tile, 0,
-                                            reinterpret_cast<StripLds<T, NS, 1> *>(lds));
+        strip_piece<T, NS, 1, kRaggedWaves, TALL>(d.sg, vp, bin_start + d.bin_off,
+                                                  gu - d.unit_off, sub, coef, beta, horner, tile, 0,
+                                                  reinterpret_cast<StripLds<T, NS, 1, TALL> *>(lds));
 }
 
 // Ragged form of strip_reduce_kernel: heavy lists global units.
@@ -1000,13 +1002,15 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
     const int64_t line = std::min<int64_t>(
         std::max<int64_t>((int64_t)sg.nunits * ntr, 512) / (narrow64 ? 2 : 4), narrow64 ? 2048 : 1024);
     constexpr int kPieceWaves = 4;
+    const bool tall = sg.H > strip_short_rows(sg.ns);
     const int waves =
-        even >= line && ub <= UINT32_MAX / (kStripLanes * kPieceWaves) ? kPieceWaves : 1;
+        !tall && even >= line && ub <= UINT32_MAX / (kStripLanes * kPieceWaves) ? kPieceWaves : 1;
     const T b = (T)beta;
     JFA_DISPATCH_NS(sg.ns, {
         if (phases & kStripSpread) {
-            auto kernel = waves > 1 ? spread_strip_kernel<T, NS_, kPieceWaves>
-                                    : spread_strip_kernel<T, NS_, 1>;
+            auto kernel = waves > 1 ? spread_strip_kernel<T, NS_, kPieceWaves, false>
+                          : tall    ? spread_strip_kernel<T, NS_, 1, (NS_ <= 8)>
+                                    : spread_strip_kernel<T, NS_, 1, false>;
             kernel<<<dim3(grid, ntr), kStripLanes * waves, 0, stream>>>(
                 sg, pts, bin_start, piece_start, npieces, piece_unit, coef, b, kerevalmeth,
                 pack_stride, scratch, scratch_stride);
@@ -1062,10 +1066,13 @@ int launch_ragged_strip(const RaggedLaunch &rl, const StripPts<T> &pts, const T 
     const unsigned grid = (unsigned)ub;
     const T b = (T)beta;
     JFA_DISPATCH_NS(rl.ns, {
-        if (phases & kStripSpread)
-            ragged_strip_kernel<T, NS_><<<grid, kStripLanes * kRaggedWaves, 0, stream>>>(
+        if (phases & kStripSpread) {
+            auto kernel = rl.tall ? ragged_strip_kernel<T, NS_, (NS_ <= 8)>
+                                  : ragged_strip_kernel<T, NS_, false>;
+            kernel<<<grid, kStripLanes * kRaggedWaves, 0, stream>>>(
                 rl.virt, rl.unit_virt, pts, rl.bin_start, rl.piece_start, rl.npieces,
                 rl.piece_unit, coef, b, kerevalmeth, rl.ptrs, rl.nprob, scratch_all);
+        }
         if (phases & kStripMerge) {
             const int64_t rb = rl.max_heavy * rl.reduce_chunks;
             ragged_reduce_kernel<T, NS_><<<(unsigned)(rb < 2048 ? rb : 2048), 256, 0, stream>>>(

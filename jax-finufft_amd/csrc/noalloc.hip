@@ -186,7 +186,8 @@ int run_noalloc(jfa_stream_t stream_, float eps, int64_t iflag, int64_t n_tot, i
                   (long long)g.nf[0], (long long)g.nf[1], 2 * g.ns);
         return JFA_ERR_NOT_SUPPORTED;
     }
-    const StripGeom sg = strip_geometry(g, kStripPiece);
+    StripGeom sg = strip_geometry(g, kStripPiece);
+    strip_units(sg, n_j, 1, 0);
 
     // sizes first, against the array's capacity
     Carve count{nullptr};

@@ -192,12 +192,7 @@ bool jfa::strip_applicable(jfa_plan p) {
     return ((nz * strips * g.nf[1] + 1) << kStripKeyShift) <= (int64_t)UINT32_MAX;
 }
 
-// Strip geometry and bins for the strip spreader.  Units are as tall as the
-// spreading kernel's accumulators allow (strip_row_tiles of 16 rows hold H +
-// ns - 1; 9 rows for every ns <= 8): shorter ones only add tile overlap, since a
-// unit's points are spread at the same cost whatever its height.  H stays within
-// [ns, nf1 - ns + 1] so that a cell is covered by at most two units per axis.
-jfa::StripGeom jfa::strip_geometry(GridGeom &g, int pmax, int rows) {
+jfa::StripGeom jfa::strip_geometry(GridGeom &g, int pmax) {
     StripGeom sg{};
     const int ns = g.ns;
     sg.nf0 = g.nf[0];
@@ -206,13 +201,7 @@ jfa::StripGeom jfa::strip_geometry(GridGeom &g, int pmax, int rows) {
     sg.nz = g.dim == 3 ? (int)g.nf[2] : 1;
     sg.SW = 64 - ns + 1;
     sg.S = (int)((g.nf[0] + sg.SW - 1) / sg.SW);
-    const int64_t most = ns <= 8 ? 9 : 33 - ns;
-    int64_t H = rows > 0 ? std::min<int64_t>(rows, most) : most;  // rows: gpu_binsizey
-    if (H > g.nf[1] - ns + 1) H = g.nf[1] - ns + 1;
-    if (H < ns) H = ns;
-    sg.H = (int)H;
-    sg.K = (int)((g.nf[1] + H - 1) / H);
-    sg.nunits = sg.nz * sg.S * sg.K;
+    strip_set_rows(sg, strip_short_rows(ns));
     sg.pmax = pmax > 0 ? pmax : kStripPiece;
     // bins: (slice, strip, exact row), rows fastest
     g.bs[0] = sg.SW;
@@ -221,24 +210,53 @@ jfa::StripGeom jfa::strip_geometry(GridGeom &g, int pmax, int rows) {
     g.nb[0] = sg.S;
     g.nb[1] = (int)g.nf[1];
     g.nb[2] = sg.nz;
-    g.nbins = (int64_t)sg.nz * g.nb[0] * g.nb[1];
+    g.nbins = (int64_t)sg.nz * sg.S * g.nf[1];
     g.ymajor = 1;
-    // sort keys also carry the first tap's column within the strip
     g.keyshift = kStripKeyShift;
     return sg;
+}
+
+// H within [ns, nf1 - ns + 1], so that a cell is covered by at most two units per axis.
+void jfa::strip_set_rows(StripGeom &sg, int64_t rows) {
+    int64_t H = std::min<int64_t>(rows, strip_tall_rows(sg.ns));
+    H = std::max<int64_t>(std::min<int64_t>(H, sg.nf1 - sg.ns + 1), sg.ns);
+    sg.H = (int)H;
+    sg.K = (int)((sg.nf1 + H - 1) / H);
+    sg.nunits = sg.nz * sg.S * sg.K;
+}
+
+// Tall units where the short ones hold few points and are many: a unit writes its whole
+// tile and the merge reads it, 2.0 cells per grid cell in short units of ns = 8, 1.4 in
+// tall ones, whose products cost twice as much per point and whose waves are fewer.
+// Points of an even short unit, short / tall, spreading + merge, ns = 8: 131,000 units of
+// 8 826 / 543 us in fp32, 1242 / 879 in fp64; 262,000 of 30 1700 / 1349 and 2698 / 2162;
+// 37,000 of 64 272 / 274 and 423 / 427; 8208 of 12 51 / 44 and 76 / 64, of 36 56 / 61 and
+// 84 / 86; 1335 of 30 27 / 34 and 31 / 43.  Below two points most short units are empty
+// and write nothing (ns = 3 in fp64, 37,000 of one 160 / 197).
+bool jfa::strip_tall(double points, double units) {
+    const double even = points / units;
+    return even >= 2 && even < std::min(64.0, units / 400);
+}
+
+void jfa::strip_units(StripGeom &sg, int64_t M, int nb, int rows) {
+    strip_set_rows(sg, rows > 0 ? rows : strip_short_rows(sg.ns));
+    if (rows <= 0 && strip_tall((double)M * nb, (double)sg.nunits * nb))
+        strip_set_rows(sg, strip_tall_rows(sg.ns));
 }
 
 int jfa::setup_strip(jfa_plan p) {
     GridGeom &g = p->geom;
     StripGeom &sg = p->sg;
-    sg = strip_geometry(g, p->opts.gpu_maxsubprobsize, p->opts.gpu_binsizey);
-    // piece table; the tiles are sized by the point count (reserve_strip_scratch)
+    sg = strip_geometry(g, p->opts.gpu_maxsubprobsize);
+    // piece table, for the most units (of ns rows); the tiles are sized by the point count
+    // (reserve_strip_scratch)
+    const int64_t units = (int64_t)sg.nz * sg.S * ((g.nf[1] + g.ns - 1) / g.ns);
     free_ptr(reinterpret_cast<void *&>(p->d_piece_start));
-    JFA_HIP_CHECK(hipMalloc(&p->d_piece_start, sizeof(int) * (sg.nunits + 1)));
+    JFA_HIP_CHECK(hipMalloc(&p->d_piece_start, sizeof(int) * (units + 1)));
     if (!p->d_npieces) JFA_HIP_CHECK(hipMalloc(&p->d_npieces, sizeof(int) * 4));
     free_ptr(reinterpret_cast<void *&>(p->d_strip_blocksum));
     JFA_HIP_CHECK(hipMalloc(&p->d_strip_blocksum,
-                            sizeof(int) * (2 * ((sg.nunits + 255) / 256) + 2)));
+                            sizeof(int) * (2 * ((units + 255) / 256) + 2)));
     return JFA_OK;
 }
 
@@ -690,6 +708,9 @@ int jfa::default_maxsub(jfa_plan p) {
 // leave the GPU idle are split into 512 pieces, down to 256 points (10,000 fp64 points
 // on 16 x 24 modes, 3 units: 330 -> 123 us a call).
 static void size_chunks(jfa_plan p, int64_t M) {
+    const int64_t Mq = p->dim == 3 ? M * p->geom.ns : M;
+    if (p->method == JFA_METHOD_STRIP)
+        strip_units(p->sg, Mq, p->batch, p->opts.gpu_binsizey);
     if (p->opts.gpu_maxsubprobsize > 0) return;
     auto chunk = [](int64_t v, int64_t most) {
         return (int)std::min(most, std::max<int64_t>(256, (v + 63) / 64 * 64));
@@ -697,7 +718,6 @@ static void size_chunks(jfa_plan p, int64_t M) {
     const int full = default_maxsub(p);
     p->maxsub = std::max(p->geom.nbins, M / full) < 512 ? chunk(M * p->batch / 2048, full) : full;
     if (p->method == JFA_METHOD_STRIP) {
-        const int64_t Mq = p->dim == 3 ? M * p->geom.ns : M;
         const int64_t all = Mq * p->batch;
         p->sg.pmax = chunk(std::max(std::min(2 * Mq / p->sg.nunits, all / 512), all / 4096),
                            kStripPiece);

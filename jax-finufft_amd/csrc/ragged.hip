@@ -160,6 +160,7 @@ int layout(jfa_ragged r) {
     r->probs.assign(np, RaggedProb{});
     r->moff.assign(np + 1, 0);
     std::vector<StripGeom> sg(np);
+    double units = 0, unit_points = 0;  // over every transform, units short
     int64_t bins = 0;
     for (int i = 0; i < np; ++i) {
         GridGeom &g = r->probs[i].g;
@@ -181,12 +182,20 @@ int layout(jfa_ragged r) {
                       (long long)kMaxFineCells);
             return JFA_ERR_TOO_LARGE;
         }
-        sg[i] = strip_geometry(g, r->opts.gpu_maxsubprobsize, r->opts.gpu_binsizey);
+        sg[i] = strip_geometry(g, r->opts.gpu_maxsubprobsize);
+        if (r->opts.gpu_binsizey > 0) strip_set_rows(sg[i], r->opts.gpu_binsizey);
+        units += (double)sg[i].nunits * r->ntr[i];
+        unit_points += (double)r->npts[i] * r->ntr[i];
         r->probs[i].moff = r->moff[i];
         r->probs[i].bin_off = bins;
         r->moff[i + 1] = r->moff[i] + r->npts[i];
         bins += g.nbins;
     }
+    // one height for the batch, whose units share one launch
+    if (r->opts.gpu_binsizey <= 0 && strip_tall(unit_points, units))
+        for (StripGeom &s : sg) strip_set_rows(s, strip_tall_rows(ns));
+    r->rl.tall = false;
+    for (const StripGeom &s : sg) r->rl.tall = r->rl.tall || s.H > strip_short_rows(ns);
     r->mtot = r->moff[np];
     if (r->mtot > INT_MAX) {
         set_error("ragged batch of %lld points exceeds 2^31 - 1", (long long)r->mtot);
