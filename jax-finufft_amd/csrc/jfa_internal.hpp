@@ -180,6 +180,8 @@ struct RaggedLaunch {
     int nprob, nv, ns, pmax, keyshift;
     int64_t mtot, nbins, nunits, mode_blocks;
 };
+// Transforms of a problem that one wave spreads together.
+constexpr int ragged_transforms(size_t real) { return real == 4 ? 2 : 1; }
 // Workgroups of the spreading launch, one per piece.  Every transform of a problem
 // has its own pieces, so the points of a problem with T transforms count T times
 // (mtot counts them once).

@@ -879,8 +879,13 @@ __global__ void __launch_bounds__(256)
 // Waves per piece.  Problems of all densities fill the GPU together: 64 problems of
 // up to 2e6 points, 1 to 8 transforms: the batch takes 4.70 ms, with four 6.03.
 constexpr int kRaggedWaves = 1;
+// Transforms of a problem that a wave spreads together: two in fp32, whose weights are
+// then staged once.  Two in fp64 would hold 256 registers of accumulators and leave one
+// wave a SIMD: 8 problems of 1e6 to 4e6 points, up to 6 transforms, w = 8 4.22 -> 3.40 ms a
+// batch with one, 64 of 1e4 to 2e6 7.05 -> 6.00, w = 16 13.0 -> 11.3.
 template <typename T, int NS, bool TALL>
-__global__ void __launch_bounds__(kStripLanes *kRaggedWaves, (strip_waves<T, 2>()))
+__global__ void __launch_bounds__(kStripLanes *kRaggedWaves,
+                                  (strip_waves<T, ragged_transforms(sizeof(T))>()))
     ragged_strip_kernel(const RaggedVirt *__restrict__ virt, const int *__restrict__ unit_virt,
                         StripPts<T> pts, const int *__restrict__ bin_start,
                         const int *__restrict__ piece_start, const int *__restrict__ npieces,
@@ -888,7 +893,8 @@ __global__ void __launch_bounds__(kStripLanes *kRaggedWaves, (strip_waves<T, 2>(
                         const T *__restrict__ coef, T beta, int horner,
                         const void *const *__restrict__ ptrs, int nprob,
                         T *__restrict__ scratch_all) {
-    __shared__ StripLds<T, NS, 2, TALL> lds[kRaggedWaves];
+    constexpr int NT = ragged_transforms(sizeof(T));
+    __shared__ StripLds<T, NS, NT, TALL> lds[kRaggedWaves];
     const int piece = blockIdx.x;  // one workgroup per piece
     if (piece >= *npieces) return;
     const int gu = piece_unit[piece];
@@ -903,8 +909,8 @@ __global__ void __launch_bounds__(kStripLanes *kRaggedWaves, (strip_waves<T, 2>(
     vp.idx_off = d.moff;
     const int64_t tile_cells = (int64_t)(d.sg.H + NS - 1) * kStripLanes;
     T *tile = scratch_all + 2 * (d.tile_off + (piece - piece_start[d.unit_off]) * tile_cells);
-    if (d.nt > 1)
-        strip_piece<T, NS, 2, kRaggedWaves, TALL>(d.sg, vp, bin_start + d.bin_off,
+    if (NT > 1 && d.nt > 1)
+        strip_piece<T, NS, NT, kRaggedWaves, TALL>(d.sg, vp, bin_start + d.bin_off,
                                                    gu - d.unit_off, sub, coef, beta, horner, tile,
                                                    2 * d.tile_next, lds);
     else

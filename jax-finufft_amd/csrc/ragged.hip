@@ -153,6 +153,13 @@ struct DeviceScope {
     }
 };
 
+// Transforms that the wave of transform t of problem i spreads: in fp32 t and t + 1
+// share the points, and the wave of t + 1 does nothing.
+int wave_transforms(jfa_ragged r, int i, int t) {
+    if (ragged_transforms(r->is_double ? 8 : 4) == 1) return 1;
+    return (t & 1) ? 0 : (t + 1 < r->ntr[i] ? 2 : 1);
+}
+
 // Problem geometry, virtual problems, offsets; host only.
 int layout(jfa_ragged r) {
     const int ns = r->kp.ns;
@@ -240,8 +247,7 @@ int layout(jfa_ragged r) {
             v.sg = sg[i];
             v.prob = i;
             v.t = t;
-            // transforms t and t + 1 share the points: one wave spreads both
-            v.nt = (t & 1) ? 0 : (t + 1 < r->ntr[i] ? 2 : 1);
+            v.nt = wave_transforms(r, i, t);
             v.tile_next = strip_max_pieces(sg[i], r->npts[i]) * strip_tile_cells(sg[i]);
             v.m = r->npts[i];
             v.bin_off = r->probs[i].bin_off;
@@ -322,7 +328,7 @@ int check_layout(jfa_ragged r) {
         if (v.prob < 0 || v.prob >= np || v.t < 0 || v.t >= r->ntr[v.prob]) return bad("virtual problem index", v.prob, v.t);
         const GridGeom &g = r->probs[v.prob].g;
         const int64_t F = g.nf[0] * g.nf[1];
-        const int want_nt = (v.t & 1) ? 0 : (v.t + 1 < r->ntr[v.prob] ? 2 : 1);
+        const int want_nt = wave_transforms(r, v.prob, v.t);
         if (v.nt != want_nt) return bad("transforms per wave", v.nt, want_nt);
         if (v.m != r->npts[v.prob] || v.moff != r->moff[v.prob] || v.bin_off != r->probs[v.prob].bin_off)
             return bad("virtual problem points", v.m, r->npts[v.prob]);
