@@ -337,8 +337,15 @@ int reserve_fwt(jfa_plan p) {
     if (p->d_fwt) (void)hipFree(p->d_fwt);
     p->d_fwt = nullptr;
     p->fwt_bytes = 0;
-    if (hipMalloc(&p->d_fwt, bytes) != hipSuccess) {
+    hipError_t e = hipMalloc(&p->d_fwt, bytes);
+    if (e != hipSuccess) {
         (void)hipGetLastError();
+        release_strip_scratch(p);  // idle by now
+        e = hipMalloc(&p->d_fwt, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        p->d_fwt = nullptr;
         set_error("could not allocate %zu bytes for the pruned FFT", bytes);
         return JFA_ERR_ALLOC;
     }

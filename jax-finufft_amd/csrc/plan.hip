@@ -181,6 +181,9 @@ struct DeviceGuard {
 // tiles are up to seven times the grid, so only up to kNarrowRows rows (at most 2 GB
 // of tiles in fp32, 4 in fp64 for one transform).
 static constexpr int64_t kNarrowRows = 1 << 20;
+// And only up to this much memory for keys, records and tiles, which in
+// 3D are w times the points (fp32 at w = 8: 16.7 million points).
+static constexpr size_t kNarrowBytes = (size_t)8 << 30;
 bool jfa::strip_applicable(jfa_plan p) {
     const GridGeom &g = p->geom;
     if (p->dim < 2 || g.nf[0] < 2 * g.ns || g.nf[1] < 2 * g.ns) return false;
@@ -260,35 +263,100 @@ int jfa::setup_strip(jfa_plan p) {
     return JFA_OK;
 }
 
-// One scratch tile per piece of M points, for each transform of a batch.
-static int reserve_strip_scratch(jfa_plan p, int64_t M) {
-    const StripGeom &sg = p->sg;
-    if (strip_max_heavy(sg, M) + 1 > p->heavy_cap) {
+// Buffers of the strip spreader for up to M points and one transform.  Neither the piece
+// size (size_chunks) nor the unit height (strip_units) grows evenly with M, and a plan
+// that holds the buffers of M points takes fewer without allocating (a captured call must
+// not), so this bounds every count up to M: pieces of the most units, and one more per
+// piece size, of which size_chunks allows 4096 points, or 256 and at most 4096 pieces of
+// the batch or half the units' number (512 pieces of the batch).
+struct StripNeed {
+    int64_t pieces, heavy;
+    size_t tile_bytes, pack_bytes;  // per transform
+};
+static StripNeed strip_need(jfa_plan p, int64_t M) {
+    const size_t real = p->is_double ? 8 : 4;
+    const int rows = p->opts.gpu_binsizey;
+    StripGeom low = p->sg, tall = p->sg;
+    strip_set_rows(low, rows > 0 ? rows : strip_short_rows(low.ns));
+    strip_set_rows(tall, rows > 0 ? rows : strip_tall_rows(tall.ns));
+    int64_t more;
+    if (p->opts.gpu_maxsubprobsize > 0) {
+        more = M / p->opts.gpu_maxsubprobsize;
+    } else {
+        const int64_t nb = p->batch;
+        more = std::min(std::min(M / 256, 4096 / nb), std::max<int64_t>(low.nunits / 2, 512 / nb));
+        more = std::max(M / kStripPiece, more + more / 64) + 2;  // (sizes are rounded)
+    }
+    StripNeed n;
+    n.pieces = std::min<int64_t>(low.nunits, M) + more;
+    n.heavy = more + 1;
+    const int64_t cells = std::max(n.pieces * strip_tile_cells(low),
+                                   (std::min<int64_t>(tall.nunits, M) + more) *
+                                       strip_tile_cells(tall));
+    n.tile_bytes = (size_t)cells * 2 * real;
+    n.pack_bytes = (size_t)M * 4 * real;
+    return n;
+}
+
+void jfa::release_strip_scratch(jfa_plan p) {
+    free_ptr(p->d_strip_scratch);
+    free_ptr(p->d_pack);
+    p->strip_scratch_bytes = p->pack_bytes = 0;
+}
+
+// Tiles for every piece of M points and a record (c, tx, ty) per point, for as many
+// transforms at a time as there is memory for, up to `most`.
+static int reserve_strip_scratch(jfa_plan p, int64_t M, int most) {
+    const StripNeed n = strip_need(p, M);
+    p->strip_scratch_stride = strip_max_pieces(p->sg, M) * strip_tile_cells(p->sg);
+    if (n.heavy + 1 > p->heavy_cap) {
         free_ptr(reinterpret_cast<void *&>(p->d_heavy));
         p->heavy_cap = 0;
-        JFA_HIP_CHECK(hipMalloc(&p->d_heavy, sizeof(int) * (strip_max_heavy(sg, M) + 1)));
-        p->heavy_cap = strip_max_heavy(sg, M) + 1;
+        JFA_HIP_CHECK(hipMalloc(&p->d_heavy, sizeof(int) * (n.heavy + 1)));
+        p->heavy_cap = n.heavy + 1;
     }
-    if (strip_max_pieces(sg, M) > p->piece_unit_cap) {
+    if (n.pieces > p->piece_unit_cap) {
         free_ptr(reinterpret_cast<void *&>(p->d_piece_unit));
         p->piece_unit_cap = 0;
-        JFA_HIP_CHECK(hipMalloc(&p->d_piece_unit, sizeof(int) * strip_max_pieces(sg, M)));
-        p->piece_unit_cap = strip_max_pieces(sg, M);
+        JFA_HIP_CHECK(hipMalloc(&p->d_piece_unit, sizeof(int) * n.pieces));
+        p->piece_unit_cap = n.pieces;
     }
-    p->strip_scratch_stride = strip_max_pieces(sg, M) * strip_tile_cells(sg);
-    const size_t bytes =
-        (size_t)p->batch * p->strip_scratch_stride * 2 * (p->is_double ? 8 : 4);
-    if (bytes > p->strip_scratch_bytes) {
-        free_ptr(p->d_strip_scratch);
-        p->strip_scratch_bytes = 0;
-        if (hipMalloc(&p->d_strip_scratch, bytes) != hipSuccess) {
+    auto grow = [](void *&q, size_t &have, size_t want) {
+        if (want <= have) return true;
+        free_ptr(q);
+        have = 0;
+        if (hipMalloc(&q, want) != hipSuccess) {
             (void)hipGetLastError();
-            set_error("could not allocate %zu bytes of strip scratch", bytes);
+            q = nullptr;
+            return false;
+        }
+        have = want;
+        return true;
+    };
+    int k = std::min(most, p->strip_batch_most);
+    if (p->geom.nf[0] < 64)
+        while (k > 1 && k * (n.tile_bytes + n.pack_bytes) > kNarrowBytes) k = (k + 1) / 2;
+    for (bool last = false;;) {
+        if (grow(p->d_strip_scratch, p->strip_scratch_bytes, k * n.tile_bytes) &&
+            grow(p->d_pack, p->pack_bytes, k * n.pack_bytes)) {
+            p->strip_batch = k;
+            return JFA_OK;
+        }
+        release_strip_scratch(p);
+        if (k > 1) {
+            p->strip_batch_most = k = (k + 1) / 2;
+        } else if (!last) {
+            // the FFT's buffers are idle while points are spread
+            last = true;
+            free_ptr(p->d_fwt);
+            free_ptr(p->d_fft_work);
+            p->fwt_bytes = p->fft_work_bytes = 0;
+        } else {
+            set_error("could not allocate %zu bytes of strip tiles and records",
+                      n.tile_bytes + n.pack_bytes);
             return JFA_ERR_ALLOC;
         }
-        p->strip_scratch_bytes = bytes;
     }
-    return JFA_OK;
 }
 
 // ------------------------------------------------------------------ fft
@@ -300,7 +368,11 @@ static int grow_fft_work(jfa_plan p, rocfft_plan plan) {
     if (ws > p->fft_work_bytes) {
         free_ptr(p->d_fft_work);
         p->fft_work_bytes = 0;
-        JFA_HIP_CHECK(hipMalloc(&p->d_fft_work, ws));
+        if (hipMalloc(&p->d_fft_work, ws) != hipSuccess) {
+            (void)hipGetLastError();
+            release_strip_scratch(p);  // idle by now
+            JFA_HIP_CHECK(hipMalloc(&p->d_fft_work, ws));
+        }
         p->fft_work_bytes = ws;
     }
     return JFA_OK;
@@ -727,27 +799,36 @@ static void size_chunks(jfa_plan p, int64_t M) {
 // Grow the point-dependent scratch to hold M points.
 int jfa::reserve_points(jfa_plan p, int64_t M) {
     const size_t real = p->is_double ? 8 : 4;
+    auto get = [](auto *&q, size_t bytes) {
+        if (hipMalloc(&q, bytes) == hipSuccess) return true;
+        (void)hipGetLastError();
+        q = nullptr;
+        set_error("could not allocate %zu bytes for the sorted points", bytes);
+        return false;
+    };
     if (p->geom.nbins + 1 > p->cap_bins) {
+        p->cap_bins = 0;
         for (int **q : {&p->d_bin_start, &p->d_sub_start})
             free_ptr(reinterpret_cast<void *&>(*q));
         const size_t nb = (size_t)p->geom.nbins + 1;
-        JFA_HIP_CHECK(hipMalloc(&p->d_bin_start, sizeof(int) * nb));
         // the subproblem prefix, then the block sums of its scan
-        JFA_HIP_CHECK(hipMalloc(&p->d_sub_start, sizeof(int) * (nb + 2 * ((nb + 255) / 256) + 2)));
-        if (!p->d_nsub) JFA_HIP_CHECK(hipMalloc(&p->d_nsub, sizeof(int) * 4));
+        if (!get(p->d_bin_start, sizeof(int) * nb) ||
+            !get(p->d_sub_start, sizeof(int) * (nb + 2 * ((nb + 255) / 256) + 2)))
+            return JFA_ERR_ALLOC;
+        if (!p->d_nsub && !get(p->d_nsub, sizeof(int) * 4)) return JFA_ERR_ALLOC;
         p->cap_bins = (int64_t)nb;
     }
     if (M > p->cap_M) {
+        p->cap_M = 0;
         for (void **q : {(void **)&p->d_idx, (void **)&p->d_l0, (void **)&p->d_key_in,
                          (void **)&p->d_key_out, &p->d_t, &p->d_sort_temp})
             free_ptr(*q);
         const int64_t cap = std::max<int64_t>(M, 1);
-        JFA_HIP_CHECK(hipMalloc(&p->d_idx, sizeof(int) * cap));
-        JFA_HIP_CHECK(hipMalloc(&p->d_l0, sizeof(int) * cap * p->dim));
-        JFA_HIP_CHECK(hipMalloc(&p->d_key_in, sizeof(unsigned) * cap));
-        JFA_HIP_CHECK(hipMalloc(&p->d_key_out, sizeof(unsigned) * cap));
-        JFA_HIP_CHECK(hipMalloc(&p->d_t, real * cap * p->dim));
-        JFA_HIP_CHECK(hipMalloc(&p->d_sort_temp, radix_temp_bytes(cap)));
+        if (!get(p->d_idx, sizeof(int) * cap) || !get(p->d_l0, sizeof(int) * cap * p->dim) ||
+            !get(p->d_key_in, sizeof(unsigned) * cap) ||
+            !get(p->d_key_out, sizeof(unsigned) * cap) || !get(p->d_t, real * cap * p->dim) ||
+            !get(p->d_sort_temp, radix_temp_bytes(cap)))
+            return JFA_ERR_ALLOC;
         p->cap_M = cap;
     }
     return JFA_OK;
@@ -821,16 +902,24 @@ static int sort_points(jfa_plan p, int64_t M, const T *x, const T *y, const T *z
                                  p->maxsub, p->d_idx, p->d_l0, (T *)p->d_t, p->stream);
 }
 
-// Auto method for 3D spreading, once the point count is known.  The strip
-// spreader sorts ns slice points per point, so it needs M * ns < 2^31 (about
-// 28 ns bytes of keys and records per point); above that the LDS-tile or
-// global method spreads instead, with the plan's ordinary bins.  An explicit
+// Auto method for spreading, once the point count is known.  In 3D the strip spreader
+// sorts ns slice points per point, so it needs M * ns < 2^31; grids narrower than a strip
+// have a bound on its memory (kNarrowBytes), others what the device has.  Above that the
+// LDS-tile or global method spreads instead, with the plan's ordinary bins.  An explicit
 // gpu_method is never changed.
-static int choose_3d_spread_method(jfa_plan p, int64_t M) {
-    if (p->dim != 3 || p->type == 2 || p->opts.gpu_method != JFA_METHOD_AUTO) return JFA_OK;
+static int choose_spread_method(jfa_plan p, int64_t M) {
+    if (p->dim < 2 || p->type == 2 || p->opts.gpu_method != JFA_METHOD_AUTO) return JFA_OK;
     GridGeom &g = p->geom;
-    const bool fits = M * (int64_t)g.ns <= (int64_t)INT_MAX;
-    const bool want_strip = fits && strip_applicable(p);
+    bool want_strip = strip_applicable(p) && M <= p->strip_most_M;
+    const int64_t Mq = p->dim == 3 ? M * (int64_t)g.ns : M;
+    if (p->dim == 3) want_strip = want_strip && Mq <= (int64_t)INT_MAX;
+    if (want_strip && g.nf[0] < 64) {
+        // keys, indices and their sort's scratch, first taps and Horner variables, records
+        // and tiles (of which a narrow grid has few)
+        const size_t real = p->is_double ? 8 : 4;
+        const size_t per_point = 4 * 3 + 12 + (4 + real) * p->dim + 4 * real;
+        want_strip = (size_t)Mq * per_point <= kNarrowBytes;
+    }
     if (want_strip == (p->method == JFA_METHOD_STRIP)) return JFA_OK;
     if (want_strip) {
         if (int rc = setup_strip(p)) return rc;
@@ -851,26 +940,36 @@ int jfa::setpts_12(jfa_plan p, int64_t M, const void *x, const void *y, const vo
         set_error("number of points %lld outside [0, 2^31)", (long long)M);
         return JFA_ERR_TOO_LARGE;
     }
-    if (int rc = choose_3d_spread_method(p, M)) return rc;
     const void *xs[3] = {x, y, z};
     for (int d = 0; d < p->dim; ++d)
         if (M > 0 && !xs[d]) {
             set_error("points for dimension %d are NULL", d);
             return JFA_ERR_BAD_ARG;
         }
-    // the 3D strip spreader sorts ns slice points per point
-    const int64_t sorted_count =
-        p->method == JFA_METHOD_STRIP && p->dim == 3 ? M * p->geom.ns : M;
-    if (sorted_count > INT_MAX) {
-        set_error("%lld points make %lld slice points, beyond 2^31 - 1 (use gpu_method 1 or 2)",
-                  (long long)M, (long long)sorted_count);
-        return JFA_ERR_TOO_LARGE;
+    for (;;) {
+        if (int rc = choose_spread_method(p, M)) return rc;
+        // the 3D strip spreader sorts ns slice points per point
+        const bool strips = p->method == JFA_METHOD_STRIP;
+        const int64_t sorted_count = strips && p->dim == 3 ? M * p->geom.ns : M;
+        if (sorted_count > INT_MAX) {
+            set_error("%lld points make %lld slice points, beyond 2^31 - 1 (use gpu_method 1 or 2)",
+                      (long long)M, (long long)sorted_count);
+            return JFA_ERR_TOO_LARGE;
+        }
+        int rc = reserve_points(p, sorted_count);
+        if (rc == JFA_OK) {
+            p->M = M;
+            if (M == 0) return JFA_OK;
+            size_chunks(p, M);
+            if (strips && p->type == 1) rc = reserve_strip_scratch(p, sorted_count, p->batch);
+        }
+        if (rc == JFA_OK) break;
+        if (rc != JFA_ERR_ALLOC || !strips || M < 1 || p->opts.gpu_method != JFA_METHOD_AUTO)
+            return rc;
+        // no memory for strips: by LDS tiles
+        release_strip_scratch(p);
+        p->strip_most_M = M - 1;
     }
-    int rc = reserve_points(p, sorted_count);
-    if (rc) return rc;
-    p->M = M;
-    if (M == 0) return JFA_OK;
-    size_chunks(p, M);
     if (p->is_double)
         return sort_points<double>(p, M, (const double *)x, (const double *)y,
                                    (const double *)z);
@@ -940,23 +1039,12 @@ static int spread_timed(jfa_plan p, const T *c, int64_t c_stride, T *fw, int64_t
     if (M == 0) return launch_fill_zero(fw, (int64_t)sizeof(T) * 2 * fw_stride * ntr, p->stream);
     // points the spreader walks: M, or the ns slice points of each in 3D
     const int64_t Mq = p->dim == 3 ? M * p->geom.ns : M;
-    if (int rc = reserve_strip_scratch(p, Mq)) return rc;
-    // one record (c, tx, ty) per point and transform of a batch: the spreader's
-    // only scattered read
-    const size_t pack_bytes = (size_t)std::min(p->batch, ntr) * Mq * 4 * sizeof(T);
-    if (pack_bytes > p->pack_bytes) {
-        free_ptr(p->d_pack);
-        if (hipMalloc(&p->d_pack, pack_bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            p->pack_bytes = 0;
-            set_error("could not allocate %zu bytes of spreading records", pack_bytes);
-            return JFA_ERR_ALLOC;
-        }
-        p->pack_bytes = pack_bytes;
-    }
+    // (with one record (c, tx, ty) per point and transform: the spreader's only
+    // scattered read)
+    if (int rc = reserve_strip_scratch(p, Mq, std::min(p->batch, ntr))) return rc;
     const StripPts<T> pts{Mq, p->d_idx, p->d_key_out, (const T *)p->d_pack, nullptr, nullptr, 0, 0};
-    for (int t0 = 0; t0 < ntr; t0 += p->batch) {
-        const int nb = std::min(p->batch, ntr - t0);
+    for (int t0 = 0; t0 < ntr; t0 += p->strip_batch) {
+        const int nb = std::min(p->strip_batch, ntr - t0);
         const int rc =
             p->dim == 3
                 ? launch_strip3_pack<T>(c + 2 * t0 * c_stride, c_stride, (const T *)p->d_t,

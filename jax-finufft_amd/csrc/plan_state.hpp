@@ -1,6 +1,7 @@
 // The plan object behind the opaque jfa_plan handle.
 #pragma once
 
+#include <climits>
 #include <map>
 #include <utility>
 #include <string>
@@ -68,7 +69,7 @@ struct jfa_plan_s {
     // 2D strip spreader
     jfa::StripGeom sg{};
     int *d_piece_start = nullptr, *d_npieces = nullptr;
-    int *d_piece_unit = nullptr;  // unit of every piece, strip_max_pieces(sg, M) entries
+    int *d_piece_unit = nullptr;  // unit of every piece
     int64_t piece_unit_cap = 0;
     int *d_heavy = nullptr;       // [count, crowded units], 1 + strip_max_heavy(sg, M)
     int64_t heavy_cap = 0;
@@ -76,8 +77,13 @@ struct jfa_plan_s {
     void *d_strip_scratch = nullptr;
     size_t strip_scratch_bytes = 0;
     int64_t strip_scratch_stride = 0;  // complex cells per transform
-    void *d_pack = nullptr;            // batch x M records (c, tx, ty)
+    void *d_pack = nullptr;            // strip_batch x M records (c, tx, ty)
     size_t pack_bytes = 0;
+    int strip_batch = 1;               // transforms spread at a time: the batch, or as many as
+                                       // there was memory for
+    int strip_batch_most = INT_MAX;    // (found by a failed allocation)
+    int64_t strip_most_M = INT64_MAX;  // point counts up to which auto spreads by strips
+                                       // (there was no memory for more)
 
     // type 3
     jfa_plan inner = nullptr;     // type-2 plan from the spread grid to the targets
@@ -132,6 +138,8 @@ template <typename T>
 int axis_grid_to_modes(jfa_plan p, T *fw, T *work, T *fk, int nb);
 template <typename T>
 int axis_modes_to_grid(jfa_plan p, const T *fk, T *work, T *fw, int nb);
+// Gives back the spreader's tiles and records; the next call allocates them again.
+void release_strip_scratch(jfa_plan p);
 bool strip_applicable(jfa_plan p);
 int setup_strip(jfa_plan p);
 int upload_kernel_tables(jfa_plan p, const int64_t *nmodes_for_dk);

@@ -1,0 +1,106 @@
+"""What the strip spreader does when its keys, records and tiles are many: a bound on
+narrow grids, fewer transforms at a time and then LDS tiles where the device has no room.
+Memory is filled by a tensor of the test; what is left is many times what the kernels
+that run need."""
+
+import contextlib
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import cnormal, dev, host, rel_l2, uniform_points
+from jax_finufft_amd._native import Plan
+
+pytestmark = pytest.mark.gpu
+
+TILES, STRIPS = 2, 3
+GIB = 1 << 30
+
+
+def _method(plan):
+    return plan.setpts_info()["method"]
+
+
+@contextlib.contextmanager
+def _memory_left(nbytes):
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    free, _ = torch.cuda.mem_get_info()
+    filler = torch.empty(max(0, free - nbytes), dtype=torch.uint8, device="cuda")
+    try:
+        yield
+    finally:
+        torch.cuda.synchronize()
+        del filler
+        torch.cuda.empty_cache()
+
+
+def _run(plan, x, c, shape):
+    out = torch.empty(shape, dtype=torch.complex64, device="cuda")
+    plan.setpts(*x)
+    plan.execute(c, out)
+    torch.cuda.synchronize()
+    return out
+
+
+def test_narrow_grid_memory_is_bounded():
+    # 24^3 modes, 48^3 cells, width 8: eight slice points of 64 bytes per point
+    plan = Plan(1, (24, 24, 24), iflag=1, eps=1e-6, dtype=torch.complex64)
+    small, large = 1_000_000, 17_000_000
+    x = [torch.rand(large, device="cuda") for _ in range(3)]
+    plan.setpts(*[a[:small] for a in x])
+    assert _method(plan) == STRIPS
+    free, _ = torch.cuda.mem_get_info()
+    plan.setpts(*x)
+    torch.cuda.synchronize()
+    assert _method(plan) == TILES
+    assert free - torch.cuda.mem_get_info()[0] < 2 * GIB
+    plan.setpts(*[a[:small] for a in x])
+    assert _method(plan) == STRIPS
+    plan.destroy()
+
+
+def test_no_room_for_strips_spreads_by_tiles():
+    rng = np.random.default_rng(81)
+    M, modes = 6_000_000, (64, 64, 64)
+    x = [dev(a) for a in uniform_points(rng, 3, M, "f32")]
+    c = dev(cnormal(rng, M, "f32"))
+    ref = Plan(1, modes, iflag=1, eps=1e-6, dtype=torch.complex64)
+    want = host(_run(ref, x, c, modes))
+    assert _method(ref) == STRIPS
+    ref.destroy()
+    # 3 GB for strips, 0.4 GB for tiles
+    plan = Plan(1, modes, iflag=1, eps=1e-6, dtype=torch.complex64)
+    with _memory_left(2 * GIB):
+        got = host(_run(plan, x, c, modes))
+        assert _method(plan) == TILES
+    assert rel_l2(got, want) <= 2e-6
+    # fewer points take strips again
+    plan.setpts(*[a[:100_000] for a in x])
+    assert _method(plan) == STRIPS
+    plan.destroy()
+
+
+def test_no_room_for_every_transform_spreads_fewer_at_a_time():
+    rng = np.random.default_rng(82)
+    M, modes, T = 1_000_000, (1024, 1024), 24
+    x = [dev(a) for a in uniform_points(rng, 2, M, "f32")]
+    c = dev(cnormal(rng, (T, M), "f32"))
+    want = torch.empty((T,) + modes, dtype=torch.complex64, device="cuda")
+    got = torch.empty_like(want)
+    ref = Plan(1, modes, iflag=1, ntransf=T, eps=1e-6, dtype=torch.complex64)
+    ref.setpts(*x)
+    ref.execute(c, want)
+    torch.cuda.synchronize()
+    ref.destroy()
+    # tiles and records of 24 transforms: about 3 GB; the FFT's buffer 0.4 GB
+    plan = Plan(1, modes, iflag=1, ntransf=T, eps=1e-6, dtype=torch.complex64)
+    with _memory_left(2 * GIB):
+        for _ in range(2):
+            plan.setpts(*x)
+            plan.execute(c, got)
+            torch.cuda.synchronize()
+        assert _method(plan) == STRIPS
+    assert torch.equal(got, want)
+    plan.destroy()
