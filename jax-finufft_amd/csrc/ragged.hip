@@ -72,8 +72,8 @@ struct jfa_ragged_s {
         rocfft_plan plan_x, plan_y;
     };
     std::vector<FftClass> fft;
-    int64_t g_cells = 0;
-    void *d_g = nullptr;  // pruned-FFT buffers [n0][nf1] per virtual problem
+    int64_t g_cells = 0;  // pruned-FFT buffers [n0][nf1] per virtual problem, in d_scratch
+                          // (written once the tiles are merged)
     rocfft_execution_info fft_info = nullptr;
     void *d_fft_work = nullptr;
     size_t fft_work_bytes = 0;
@@ -115,7 +115,6 @@ void release(jfa_ragged r) {
                      (void **)&r->d_key_out, &r->d_sort_temp, (void **)&r->d_bin_start,
                      (void **)&r->d_piece_start, (void **)&r->d_npieces,
                      (void **)&r->d_piece_unit, (void **)&r->d_heavy, &r->d_fw, &r->d_scratch,
-                     &r->d_g,
                      &r->d_fft_work, (void **)&r->d_blocksum})
         free_dev(*q);
     if (r->h_ptrs) (void)hipHostFree((void *)r->h_ptrs);
@@ -431,18 +430,12 @@ int allocate(jfa_ragged r) {
     JFA_HIP_CHECK(hipMalloc(&r->d_piece_unit, sizeof(int) * std::max<int64_t>(r->max_pieces, 1)));
     JFA_HIP_CHECK(hipMalloc(&r->d_heavy, sizeof(int) * (r->max_heavy + 1)));
     JFA_HIP_CHECK(hipMalloc(&r->d_blocksum, sizeof(int) * (2 * ((r->rl.nunits + 255) / 256) + 1)));
+    const int64_t scratch = std::max<int64_t>({r->tile_cells, r->g_cells, 1});
     if (hipMalloc(&r->d_fw, 2 * real * std::max<int64_t>(r->fw_cells, 1)) != hipSuccess ||
-        hipMalloc(&r->d_scratch, 2 * real * std::max<int64_t>(r->tile_cells, 1)) != hipSuccess) {
+        hipMalloc(&r->d_scratch, 2 * real * scratch) != hipSuccess) {
         (void)hipGetLastError();
-        set_error("could not allocate the ragged batch's fine grids (%lld cells) and tiles",
-                  (long long)r->fw_cells);
-        return JFA_ERR_ALLOC;
-    }
-
-    if (hipMalloc(&r->d_g, 2 * real * std::max<int64_t>(r->g_cells, 1)) != hipSuccess) {
-        (void)hipGetLastError();
-        set_error("could not allocate the ragged batch's pruned-FFT buffers (%lld cells)",
-                  (long long)r->g_cells);
+        set_error("could not allocate the ragged batch's fine grids (%lld cells) and tiles (%lld)",
+                  (long long)r->fw_cells, (long long)scratch);
         return JFA_ERR_ALLOC;
     }
     // per class: in-place 1D FFTs along x of every row, then along y of the
@@ -531,7 +524,7 @@ int enqueue_execute(jfa_ragged r, hipStream_t s) {
     rocfft_execution_info_set_stream(r->fft_info, s);
     for (auto &c : r->fft) {
         T *fw = (T *)r->d_fw + 2 * c.fw_off;
-        T *G = (T *)r->d_g + 2 * c.g_off;
+        T *G = (T *)r->d_scratch + 2 * c.g_off;
         void *bx[1] = {fw}, *by[1] = {G};
         rocfft_status st = rocfft_execute(c.plan_x, bx, nullptr, r->fft_info);
         if (st == rocfft_status_success) {
@@ -545,7 +538,7 @@ int enqueue_execute(jfa_ragged r, hipStream_t s) {
         }
     }
     return launch_ragged_deconv<T>(r->rl, (const T *)r->d_dk, r->opts.modeord,
-                                   (const T *)r->d_g, s);
+                                   (const T *)r->d_scratch, s);
 }
 
 template <typename T>
