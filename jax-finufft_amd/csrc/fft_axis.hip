@@ -427,6 +427,8 @@ __global__ void __launch_bounds__(256) axis_twiddle_kernel(AxisFft f, T *__restr
 constexpr int kRadices[] = {16, 15, 12, 10, 9, 8, 6, 5, 4, 3, 2};
 constexpr int kMaxThreads = 1024;
 constexpr size_t kMaxLds = 144 * 1024;
+// Most threads of one launch; larger passes (16 transforms on 1024^3 cells) take several.
+constexpr int64_t kLaunchThreads = UINT32_MAX;
 
 // The stages of length n: as few as possible, then with the largest smallest
 // radix (a stage of radix r uses n / r threads per column).
@@ -463,17 +465,18 @@ int launch_rows(const AxisFft &f, const T *tw, int64_t rows, int64_t n, int mode
     const size_t row_bytes = (size_t)padded(f.L) * 2 * sizeof(T);
     // about 256 threads per workgroup
     const int NR = std::max(1, std::min<int>(256 / P, (int)(48 * 1024 / row_bytes)));
-    const int64_t blocks = (rows + NR - 1) / NR;
-    if (blocks > INT32_MAX) {
-        set_error("FFT pass of %lld rows is too large", (long long)rows);
-        return JFA_ERR_TOO_LARGE;
-    }
     const size_t lds = NR * row_bytes;
+    const unsigned threads = (unsigned)((P * NR + 63) / 64 * 64);
+    const int64_t most = kLaunchThreads / threads * NR;  // rows of a launch
     auto go = [&](auto kernel) -> int {
         if (int rc = allow_lds(kernel, lds)) return rc;
-        kernel<<<(unsigned)blocks, (unsigned)((P * NR + 63) / 64 * 64), lds, s>>>(
-            f, P, NR, rows, (int)n, modeord, swap, tw, in, out);
-        JFA_HIP_CHECK(hipGetLastError());
+        for (int64_t r0 = 0; r0 < rows; r0 += most) {
+            const int64_t part = std::min(most, rows - r0);
+            kernel<<<(unsigned)((part + NR - 1) / NR), threads, lds, s>>>(
+                f, P, NR, part, (int)n, modeord, swap, tw, in + 2 * r0 * (TO_GRID ? n : f.L),
+                out + 2 * r0 * (TO_GRID ? f.L : n));
+            JFA_HIP_CHECK(hipGetLastError());
+        }
         return JFA_OK;
     };
     if (f.r[0] <= 8) return go(fft_rows_kernel<T, 8, TO_GRID>);
@@ -503,19 +506,24 @@ int launch_cols(const AxisFft &f, const T *tw, int64_t outer, const ColsShape &s
     if (outer == 0 || sh.inner == 0) return JFA_OK;
     const int tc = cols_per_group<T>(f, outer * sh.inner);
     const int64_t tiles = (sh.inner + tc - 1) / tc;
-    if (sh.inner > INT32_MAX || tiles * outer > INT32_MAX) {
-        set_error("FFT pass of %lld x %lld columns is too large", (long long)outer,
-                  (long long)sh.inner);
+    const unsigned threads = (unsigned)((f.P * tc + 63) / 64 * 64);
+    if (sh.inner > INT32_MAX || tiles * threads > kLaunchThreads) {
+        set_error("FFT pass of %lld columns is too large", (long long)sh.inner);
         return JFA_ERR_TOO_LARGE;
     }
     sh.tiles = (int)tiles;
     const size_t lds = f.count > 1 ? (size_t)padded(f.L) * tc * 2 * sizeof(T) : 0;
-    const unsigned blocks = (unsigned)(tiles * outer);
-    const unsigned threads = (unsigned)((f.P * tc + 63) / 64 * 64);
+    const int64_t most = kLaunchThreads / threads / tiles;  // outer indices of a launch
+    const int64_t mode_step = 2 * sh.n * sh.inner, grid_step = 2 * sh.wl * sh.inner;
     auto go = [&](auto kernel) -> int {
         if (int rc = allow_lds(kernel, lds)) return rc;
-        kernel<<<blocks, threads, lds, s>>>(f, sh, tw, dk0, dkm, dkl, in, out);
-        JFA_HIP_CHECK(hipGetLastError());
+        for (int64_t o0 = 0; o0 < outer; o0 += most) {
+            const unsigned blocks = (unsigned)(tiles * std::min(most, outer - o0));
+            kernel<<<blocks, threads, lds, s>>>(f, sh, tw, dk0, dkm, dkl,
+                                                in + o0 * (TO_GRID ? mode_step : grid_step),
+                                                out + o0 * (TO_GRID ? grid_step : mode_step));
+            JFA_HIP_CHECK(hipGetLastError());
+        }
         return JFA_OK;
     };
     auto pick = [&](auto tcc) -> int {
