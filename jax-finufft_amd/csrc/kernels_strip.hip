@@ -184,6 +184,10 @@ __device__ __forceinline__ void stage_weights(Coef coef, T beta, int horner, T t
     for (int i = 0; i < NS; ++i) out[i] = k[i];
 }
 
+// Finite, with room for its products with weights.
+__device__ __forceinline__ bool plain(float v) { return fabsf(v) <= 1e38f; }
+__device__ __forceinline__ bool plain(double v) { return fabs(v) <= 1e307; }
+
 // Order of one wave's LDS accesses: its instructions reach LDS in program order,
 // so only the compiler has to keep it.
 __device__ __forceinline__ void wave_sync() {
@@ -311,7 +315,7 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
     for (int bb = pb; bb < pe; bb += kStripLanes) {
         const int nb = min(kStripLanes, pe - bb);
         const unsigned pkey = key1;
-        const Quad<T> rq = rq1;
+        Quad<T> rq = rq1;
         Pair<T> ct[NC];
 #pragma unroll
         for (int t = 0; t < NC; ++t) ct[t] = ct1[t];
@@ -361,6 +365,19 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
         uintptr_t cf_bits = reinterpret_cast<uintptr_t>(coef);
         asm volatile("" : "+s"(cf_bits));
         const auto *cf = reinterpret_cast<const __attribute__((address_space(4))) T *>(cf_bits);
+        // Points whose values would not stay within their taps (0 x inf is NaN) go in as
+        // zeros here, and one by one below.
+        bool odd = !plain(rq.x) || !plain(rq.y) || !(fabs(rq.z) <= T(2)) || !(fabs(rq.w) <= T(2));
+#pragma unroll
+        for (int t = 1; t < NT; ++t) odd = odd || !plain(ct[t - 1].x) || !plain(ct[t - 1].y);
+        uint64_t left = __ballot(lane < nb && odd);
+        if (left && odd) {
+            rq.x = rq.y = T(0);
+            if (!(fabs(rq.z) <= T(2))) rq.z = T(0);
+            if (!(fabs(rq.w) <= T(2))) rq.w = T(0);
+#pragma unroll
+            for (int t = 1; t < NT; ++t) ct[t - 1] = Pair<T>{T(0), T(0)};
+        }
         if (lane < nb) {
             const int v0 = Sh::kGuard + lane * S;
             stage_weights<T, NS>(cf, beta, horner, rq.z, lds.kx + v0);
@@ -442,7 +459,35 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
                 });
             }
         });
-        wave_sync();
+        for (; left; left &= left - 1) {
+            const int q = __builtin_ctzll(left);
+            const unsigned key = pts.key[bb + q];
+            const int i = pts.idx[bb + q];
+            const Quad<T> p = point_record(pts, i);
+            const int qx = (int)(key & ((1u << kStripKeyShift) - 1));
+            const int qy = (int)((int64_t)(key >> kStripKeyShift) - rowbase) - r0;
+            // (a weight of NaN where the coordinate is)
+            const T u = (fabs(p.z) <= T(2) ? T(0) : p.z - p.z) + (fabs(p.w) <= T(2) ? T(0) : p.w - p.w);
+            unroll<NT>([&](auto tc) {
+                constexpr int t = decltype(tc)::value;
+                Pair<T> c{p.x, p.y};
+                if constexpr (t > 0)
+                    c = reinterpret_cast<const Pair<T> *>(pts.c + t * pts.c_tstride)[i - pts.idx_off];
+                unroll<RT * NF * 4>([&](auto ec) {
+                    constexpr int e = decltype(ec)::value, h = e / (NF * 4), f = e / 4 % NF,
+                                  r = e % 4;
+                    const int dy = 16 * h + M::row(r, g) - qy;
+                    const int dx = (f << Sh::kFrameShift) + i16 - qx;
+                    if (unsigned(dy) < NS && unsigned(dx) < NS &&
+                        (!Sh::kNarrow || f == qx >> Sh::kFrameShift)) {
+                        const int v0 = Sh::kGuard + q * S;
+                        const T w = lds.kx[v0 + dx] * lds.ky[v0 + dy] + u;
+                        re[t][h][f][r] += c.x * w;
+                        im[t][h][f][r] += c.y * w;
+                    }
+                });
+            });
+        }
     }
     // the tile's rows to scratch: value e = (t, h, r, k) is row 16 h + row(r, g),
     // column 16 k + i16 of transform t
