@@ -116,7 +116,9 @@ Buffers carve(Carve &c, const StripGeom &sg, const GridGeom &g, int64_t M, int64
     b.key_out = c.take<unsigned>(4 * m);
     b.idx = c.take<int>(4 * m);
     b.rec = c.take<float>(8 * m);
-    b.pack = c.take<float>(16 * m);
+    // the sort is done before the records are packed, and has its scratch there
+    b.pack = c.take<float>(std::max<size_t>(16 * m, radix_temp_bytes(m)));
+    b.sort_temp = b.pack;
     b.bin_start = c.take<int>(4 * (g.nbins + 1));
     b.piece_start = c.take<int>(4 * (sg.nunits + 1));
     b.npieces = c.take<int>(16);
@@ -128,9 +130,6 @@ Buffers carve(Carve &c, const StripGeom &sg, const GridGeom &g, int64_t M, int64
     b.fw = c.take<float>(8 * g.nf[0] * g.nf[1]);
     // the FFT's compact buffer is written once the tiles are merged
     b.G = b.tiles;
-    // the sort is done before the records are packed, and its scratch fits there (8
-    // bytes a point and, per 2048 points, a table of at most 4096)
-    b.sort_temp = b.pack;
     b.tw0 = c.take<float>(8 * g.nf[0]);
     b.tw1 = c.take<float>(8 * g.nf[1]);
     b.coef = c.take<float>(4 * (size_t)nc * g.ns);
