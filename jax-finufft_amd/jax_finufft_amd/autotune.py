@@ -135,8 +135,9 @@ def clear():
     _lib().jfa_tune_clear()
 
 
-# unit height (rows) x piece size for ragged batches; (0, 0) is the default rule
-RAGGED_CANDIDATES = [(0, 0), (16, 0), (32, 0), (64, 0), (0, 2048), (32, 2048), (32, 8192)]
+# unit height (rows, at most 33 - width) x piece size for ragged batches; (0, 0) is the
+# default rule
+RAGGED_CANDIDATES = [(0, 0), (16, 0), (32, 0), (0, 2048), (32, 2048), (32, 8192)]
 
 
 def tune_ragged(output_shapes, sources, points_x, points_y, iflag=1, eps=1e-6, opts=None,

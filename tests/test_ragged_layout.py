@@ -107,6 +107,20 @@ def test_random_batches(L, seed):
     assert info[0] == Ms.sum() and info[3] == Ts.sum()
 
 
+@pytest.mark.parametrize("eps", [1e-1, 1e-3, 1e-6])
+def test_tuning_candidates_differ(L, eps):
+    # dense problems, whose default units are the short ones
+    from jax_finufft_amd.autotune import RAGGED_CANDIDATES
+
+    units = []
+    for rows, pmax in RAGGED_CANDIDATES:
+        rc, info = _check(L, [(200, 300)], [2], [900_000], eps=eps, gpu_binsizey=rows,
+                          gpu_maxsubprobsize=pmax)
+        assert rc == 0, _native.last_error()
+        units.append((int(info[2]), int(info[7])))
+    assert len(set(units)) == len(units), units
+
+
 def test_bad_arguments_are_rejected(L):
     rc, _ = _check(L, [(32, 32)], [0], [10])
     assert rc == 2 and "ntransf" in _native.last_error()
