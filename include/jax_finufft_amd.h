@@ -83,7 +83,7 @@ typedef struct {
     int debug;             /* 1: print per-stage timings to stderr */
     int gpu_binsizex, gpu_binsizey, gpu_binsizez; /* LDS-tile bins; for the strip
                               method gpu_binsizey asks for the unit height in rows,
-                              of which a unit has w to 33 - w;
+                              of which a unit has w to 33 - w (to 128 where w > 8);
                               0 = default (or the autotuner's choice) */
     int gpu_maxsubprobsize;  /* points per LDS subproblem / strip piece; 0 = default */
     int gpu_spreadinterponly; /* 1: execute spreads/interpolates only; the mode

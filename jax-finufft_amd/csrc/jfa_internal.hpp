@@ -87,10 +87,10 @@ inline int64_t strip_max_pieces(const StripGeom &sg, int64_t M) {
 // Units with more than one piece hold more than pmax points each.
 inline int64_t strip_max_heavy(const StripGeom &sg, int64_t M) { return M / (sg.pmax + 1) + 1; }
 
-// Most rows of a unit that the spreading kernel's accumulators hold: short units, and
-// the tall ones of sparse grids (the same for ns > 8).
+// Most rows of a unit: short units, whose tile the spreading kernel's accumulators hold,
+// and the tall ones of sparse grids.
 constexpr int strip_short_rows(int ns) { return ns <= 8 ? 9 : 33 - ns; }
-constexpr int strip_tall_rows(int ns) { return 33 - ns; }
+constexpr int strip_tall_rows(int ns) { return ns <= 8 ? 33 - ns : 128; }
 // Strips of a grid g (nf and ns set) in short units; also sets g's bins to (strip, row),
 // rows fastest, which do not depend on the units.
 StripGeom strip_geometry(GridGeom &g, int pmax);
@@ -98,7 +98,7 @@ StripGeom strip_geometry(GridGeom &g, int pmax);
 void strip_set_rows(StripGeom &sg, int64_t rows);
 // Whether tall units suit that many points (slice points in 3D) in all of so many short
 // units, over every transform.
-bool strip_tall(double points, double units);
+bool strip_tall(int ns, double points, double units);
 // Sets the height that suits M points of nb transforms; rows > 0 asks for one
 // (gpu_binsizey).
 void strip_units(StripGeom &sg, int64_t M, int nb, int rows);

@@ -96,6 +96,7 @@ struct Mfma<double> {
 
 // Shape of a unit's tile in MFMA terms (see strip_piece).  TALL: units of more than
 // strip_short_rows rows, ns <= 8 (wider kernels' shape is always the tall one).
+constexpr bool strip_rolls(int ns, bool tall) { return tall && ns > 8; }
 template <int NS, bool TALL>
 struct StripShape {
     static constexpr bool kNarrow = NS <= 8 && !TALL;
@@ -134,12 +135,12 @@ struct StripLds {
     T kx[StripShape<NS, TALL>::kValues];
 };
 
-// The ns weights of a point along one axis to LDS, as eval_kernel computes them.  Wide
-// double kernels two taps at a time, in a loop: the accumulators leave no registers for
+// The ns weights of a point along one axis to LDS, as eval_kernel computes them.  Double
+// kernels of ns >= 8 two taps at a time, in a loop: the accumulators leave no registers for
 // every tap at once.
 template <typename T, int NS, typename Coef>
 __device__ __forceinline__ void stage_weights(Coef coef, T beta, int horner, T t, T *out) {
-    if constexpr (sizeof(T) == 8 && NS > 8) {
+    if constexpr (sizeof(T) == 8 && NS >= 8) {
         if (horner) {
             constexpr int NC = horner_nc(NS), NE = (NC + 1) / 2, NO = NC / 2, half = (NS + 1) / 2;
             const T s = t * t;
@@ -253,6 +254,13 @@ __device__ __forceinline__ PieceRange piece_range(const StripGeom &sg,
 // ns = 6 65 -> 46, 4000 points on 48 x 40 29 -> 11; 2^20 sources of a 3D type 3 at
 // ns = 8 507 -> 314.
 //
+// Tall units of ns > 8 have up to 128 rows, which the accumulators roll over: they hold
+// 32 rows, row y in place y mod 32, and whenever the points move on past the first 16
+// those are complete, go to the tile and start again at zero.  A batch is staged once and
+// multiplied window by window.  This costs registers (89 spilled) and waves; it is for
+// grids whose tiles bound the call (1e6 points on 8192^2 cells at ns = 16, units of 17
+// rows 1430 us with the merge, of 128 1150).
+//
 // W waves share a piece: each spreads a run of its points into accumulators of its
 // own, which are added through LDS in wave order at the end.
 template <typename T, int NS, int NT, int W, bool TALL>
@@ -262,6 +270,7 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
                                             T *__restrict__ tile, int64_t tile_tstride,
                                             StripLds<T, NS, NT, TALL> *lds_all) {
     using Sh = StripShape<NS, TALL>;
+    constexpr bool ROLL = strip_rolls(NS, TALL);
     using M = Mfma<T>;
     using Acc = typename M::Acc;
     constexpr int RT = Sh::kRowTiles, NF = Sh::kFrames, S = Sh::kStride;
@@ -309,186 +318,7 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
                     pts.c + t * pts.c_tstride)[i - pts.idx_off];
         }
     };
-    load_index(pb, key1, idx1);
-    load_record(pb, idx1);
-    load_index(pb + kStripLanes, key2, idx2);
-    for (int bb = pb; bb < pe; bb += kStripLanes) {
-        const int nb = min(kStripLanes, pe - bb);
-        const unsigned pkey = key1;
-        Quad<T> rq = rq1;
-        Pair<T> ct[NC];
-#pragma unroll
-        for (int t = 0; t < NC; ++t) ct[t] = ct1[t];
-        key1 = key2;
-        idx1 = idx2;
-        load_record(bb + kStripLanes, idx1);
-        load_index(bb + 2 * kStripLanes, key2, idx2);
-        const int X = (int)(pkey & ((1u << kStripKeyShift) - 1));
-        const int Y = (int)((int64_t)(pkey >> kStripKeyShift) - rowbase) - r0;
-        // this lane's slot, and the groups of four of every frame
-        constexpr int kBits = Sh::kNarrow ? 3 : 2;
-        const unsigned frame = (unsigned)X >> Sh::kFrameShift;
-        const uint64_t in = nb < kStripLanes ? (uint64_t(1) << nb) - 1 : ~uint64_t(0);
-        uint64_t bit[kBits], same = in;
-#pragma unroll
-        for (int b = 0; b < kBits; ++b) {
-            const bool one = (frame >> b) & 1;
-            bit[b] = __ballot(one);
-            same &= one ? bit[b] : ~bit[b];
-        }
-        int groups[NF];
-        uint64_t starts = 0;  // first group of every frame, 5 bits each
-        int base = 0;
-#pragma unroll
-        for (int f = 0; f < NF; ++f) {
-            uint64_t m = in;
-#pragma unroll
-            for (int b = 0; b < kBits; ++b) m &= (f >> b) & 1 ? bit[b] : ~bit[b];
-            starts |= (uint64_t)base << (5 * f);
-            groups[f] = (__popcll(m) + 3) >> 2;
-            base += groups[f];
-        }
-        const int slot = 4 * (int)((starts >> (5 * frame)) & 31) +
-                         (int)__builtin_amdgcn_mbcnt_hi(
-                             (unsigned)(same >> 32),
-                             __builtin_amdgcn_mbcnt_lo((unsigned)same, 0u));
-        bool low = true, high = false;
-        if constexpr (RT > 1) {
-            low = __builtin_amdgcn_readfirstlane(Y) < 16;
-            high = __builtin_amdgcn_readlane(Y, nb - 1) + NS > 16;
-        }
-        // (a wave's LDS writes land in order: the empty slots before the filled)
-        lds.slot[lane] = none;
-        if (lane + kStripLanes < Sh::kSlots) lds.slot[lane + kStripLanes] = none;
-        // opaque: hoisted out of the loop, the coefficients would not fit the scalar
-        // registers and spill; constant address space: scalar loads all the same
-        uintptr_t cf_bits = reinterpret_cast<uintptr_t>(coef);
-        asm volatile("" : "+s"(cf_bits));
-        const auto *cf = reinterpret_cast<const __attribute__((address_space(4))) T *>(cf_bits);
-        // Points whose values would not stay within their taps (0 x inf is NaN) go in as
-        // zeros here, and one by one below.
-        bool odd = !plain(rq.x) || !plain(rq.y) || !(fabs(rq.z) <= T(2)) || !(fabs(rq.w) <= T(2));
-#pragma unroll
-        for (int t = 1; t < NT; ++t) odd = odd || !plain(ct[t - 1].x) || !plain(ct[t - 1].y);
-        uint64_t left = __ballot(lane < nb && odd);
-        if (left && odd) {
-            rq.x = rq.y = T(0);
-            if (!(fabs(rq.z) <= T(2))) rq.z = T(0);
-            if (!(fabs(rq.w) <= T(2))) rq.w = T(0);
-#pragma unroll
-            for (int t = 1; t < NT; ++t) ct[t - 1] = Pair<T>{T(0), T(0)};
-        }
-        if (lane < nb) {
-            const int v0 = Sh::kGuard + lane * S;
-            stage_weights<T, NS>(cf, beta, horner, rq.z, lds.kx + v0);
-            stage_weights<T, NS>(cf, beta, horner, rq.w, lds.ky + v0);
-            const int ox = X & ((1 << Sh::kFrameShift) - 1);
-            StripSlot<T, NT> me;
-            me.c[0] = Pair<T>{rq.x, rq.y};
-#pragma unroll
-            for (int t = 1; t < NT; ++t) me.c[t] = ct[t - 1];
-            // narrow: byte offsets of where row 0 of the tile / column 0 of the frame
-            // lie in the staged values; wide: the first row, and lane and column
-            me.at = Sh::kNarrow
-                        ? (unsigned)((v0 - Y) * sizeof(T)) << 16 | (unsigned)((v0 - ox) * sizeof(T))
-                        : (unsigned)Y << 16 | (unsigned)(lane << 4) | (unsigned)ox;
-            lds.slot[slot] = me;
-        }
-        wave_sync();
-        // operands of the four points from slot 4 n: lane (i16, g) reads point g's
-        constexpr int NB = Sh::kNarrow ? 1 : 2;
-        struct Operands {
-            T y[RT], x[NB];
-            Pair<T> c[NT];
-        };
-        const StripSlot<T, NT> *next = lds.slot + g;
-        auto fetch = [&] {
-            Operands o;
-            const StripSlot<T, NT> s = *next;
-            next += 4;
-#pragma unroll
-            for (int t = 0; t < NT; ++t) o.c[t] = s.c[t];
-            if constexpr (Sh::kNarrow) {
-                // both halves at once (neither overflows)
-                const unsigned at = s.at + (unsigned)(i16 * sizeof(T)) * 0x10001u;
-                o.y[0] = *reinterpret_cast<const T *>(
-                    reinterpret_cast<const char *>(lds.ky) + (at >> 16));
-                o.x[0] = *reinterpret_cast<const T *>(
-                    reinterpret_cast<const char *>(lds.kx) + (at & 0xffffu));
-            } else {
-                const int ya = (int)(s.at >> 16), xa = (int)(s.at & 15u);
-                const int v0 = (int)(s.at >> 4 & 63u) * S;
-#pragma unroll
-                for (int h = 0; h < RT; ++h) {
-                    const int e = i16 + 16 * h - ya;
-                    const T v = lds.ky[v0 + (unsigned(e) < NS ? e : 0)];
-                    o.y[h] = unsigned(e) < NS ? v : T(0);
-                }
-#pragma unroll
-                for (int h = 0; h < NB; ++h) {
-                    const int e = i16 + 16 * h - xa;
-                    const T v = lds.kx[v0 + (unsigned(e) < NS ? e : 0)];
-                    o.x[h] = unsigned(e) < NS ? v : T(0);
-                }
-            }
-            return o;
-        };
-        Operands cur = fetch();
-        // frames as compile-time constants, so that the accumulators are separate
-        // registers to the compiler (as one array it copies it between frames)
-        unroll<NF>([&](auto fc) {
-            constexpr int f = decltype(fc)::value;
-            for (int n = groups[f]; n > 0; --n) {
-                const Operands o = cur;
-                cur = fetch();
-                unroll<RT>([&](auto hc) {
-                    constexpr int h = decltype(hc)::value;
-                    if (RT > 1 && !(h == 0 ? low : high)) return;
-                    const T y = o.y[h];
-                    unroll<NT>([&](auto tc) {
-                        constexpr int t = decltype(tc)::value;
-                        const T ar = y * o.c[t].x, ai = y * o.c[t].y;
-                        re[t][h][f] = M::mul(ar, o.x[0], re[t][h][f]);
-                        im[t][h][f] = M::mul(ai, o.x[0], im[t][h][f]);
-                        if constexpr (NB > 1 && f + 1 < NF) {
-                            // (no point of the last frame leaves it)
-                            re[t][h][f + 1] = M::mul(ar, o.x[NB - 1], re[t][h][f + 1]);
-                            im[t][h][f + 1] = M::mul(ai, o.x[NB - 1], im[t][h][f + 1]);
-                        }
-                    });
-                });
-            }
-        });
-        for (; left; left &= left - 1) {
-            const int q = __builtin_ctzll(left);
-            const unsigned key = pts.key[bb + q];
-            const int i = pts.idx[bb + q];
-            const Quad<T> p = point_record(pts, i);
-            const int qx = (int)(key & ((1u << kStripKeyShift) - 1));
-            const int qy = (int)((int64_t)(key >> kStripKeyShift) - rowbase) - r0;
-            // (a weight of NaN where the coordinate is)
-            const T u = (fabs(p.z) <= T(2) ? T(0) : p.z - p.z) + (fabs(p.w) <= T(2) ? T(0) : p.w - p.w);
-            unroll<NT>([&](auto tc) {
-                constexpr int t = decltype(tc)::value;
-                Pair<T> c{p.x, p.y};
-                if constexpr (t > 0)
-                    c = reinterpret_cast<const Pair<T> *>(pts.c + t * pts.c_tstride)[i - pts.idx_off];
-                unroll<RT * NF * 4>([&](auto ec) {
-                    constexpr int e = decltype(ec)::value, h = e / (NF * 4), f = e / 4 % NF,
-                                  r = e % 4;
-                    const int dy = 16 * h + M::row(r, g) - qy;
-                    const int dx = (f << Sh::kFrameShift) + i16 - qx;
-                    if (unsigned(dy) < NS && unsigned(dx) < NS &&
-                        (!Sh::kNarrow || f == qx >> Sh::kFrameShift)) {
-                        const int v0 = Sh::kGuard + q * S;
-                        const T w = lds.kx[v0 + dx] * lds.ky[v0 + dy] + u;
-                        re[t][h][f][r] += c.x * w;
-                        im[t][h][f][r] += c.y * w;
-                    }
-                });
-            });
-        }
-    }
+    int top = 0;  // rolling: the window's first row, from r0
     // the tile's rows to scratch: value e = (t, h, r, k) is row 16 h + row(r, g),
     // column 16 k + i16 of transform t
     const int rows_tile = sg.H + NS - 1;
@@ -513,15 +343,256 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
                            im[t][h][2 * k][r] + __shfl_xor(si, 8)};
         }
     };
-    auto store = [&](int e, Pair<T> v) {
-        const int t = e / (RT * 16), h = e / 16 % RT, k = e / 4 % 4, r = e % 4;
-        const int row = 16 * h + M::row(r, g);
+    auto store = [&](int e, int row, int col, Pair<T> v) {
+        const int t = e / (RT * 16), k = e / 4 % 4;
         if (row < rows_tile)
-            reinterpret_cast<Pair<T> *>(tile + t * tile_tstride)[row * kStripLanes + 16 * k + i16] =
+            reinterpret_cast<Pair<T> *>(tile + t * tile_tstride)[row * kStripLanes + 16 * k + col] =
                 v;
     };
-    if constexpr (W == 1) {
-        unroll<NT * RT * 16>([&](auto ec) { store(decltype(ec)::value, value(ec)); });
+    // Rolling: the window's first 16 rows, one row tile, are complete; they go to the
+    // tile, and the row tile starts again at zero behind the other one.
+    auto flush = [&] {
+        int ln = lane;  // opaque: addresses are computed here, not kept in registers
+        asm volatile("" : "+v"(ln));
+        auto half = [&](auto hc) {
+            constexpr int h = decltype(hc)::value;
+            // (both halves' code is alike but for the registers: kept apart)
+            asm volatile("; row tile %0" ::"n"(h));
+            unroll<NT * 16>([&](auto ec) {
+                constexpr int e0 = decltype(ec)::value, e = (e0 / 16 * RT + h) * 16 + e0 % 16;
+                store(e, top + M::row(e % 4, ln >> 4), ln & 15, value(std::integral_constant<int, e>{}));
+            });
+            asm volatile("; row tile %0 done" ::"n"(h));
+        };
+        if (top & 16)
+            half(std::integral_constant<int, RT - 1>{});
+        else
+            half(std::integral_constant<int, 0>{});
+        // (selected, in place: cleared in the branches they would be copied)
+        int odd = top & 16;
+        asm volatile("" : "+v"(odd));
+        unroll<NT * RT * NF * 4>([&](auto c) {
+            constexpr int e = decltype(c)::value, t = e / (RT * NF * 4), h = e / (NF * 4) % RT,
+                          f = e / 4 % NF, r = e % 4;
+            const bool clear = h == 0 ? odd == 0 : odd != 0;
+            re[t][h][f][r] = clear ? T(0) : re[t][h][f][r];
+            im[t][h][f][r] = clear ? T(0) : im[t][h][f][r];
+        });
+        top += 16;
+    };
+    load_index(pb, key1, idx1);
+    load_record(pb, idx1);
+    load_index(pb + kStripLanes, key2, idx2);
+    for (int bb = pb; bb < pe; bb += kStripLanes) {
+        const int nb = min(kStripLanes, pe - bb);
+        const unsigned pkey = key1;
+        Quad<T> rq = rq1;
+        Pair<T> ct[NC];
+#pragma unroll
+        for (int t = 0; t < NC; ++t) ct[t] = ct1[t];
+        key1 = key2;
+        idx1 = idx2;
+        load_record(bb + kStripLanes, idx1);
+        load_index(bb + 2 * kStripLanes, key2, idx2);
+        // opaque: hoisted out of the loop, the coefficients would not fit the scalar
+        // registers and spill; constant address space: scalar loads all the same
+        uintptr_t cf_bits = reinterpret_cast<uintptr_t>(coef);
+        asm volatile("" : "+s"(cf_bits));
+        const auto *cf = reinterpret_cast<const __attribute__((address_space(4))) T *>(cf_bits);
+        // Points whose values would not stay within their taps (0 x inf is NaN) go in as
+        // zeros here, and one by one below.
+        bool odd = !plain(rq.x) || !plain(rq.y) || !(fabs(rq.z) <= T(2)) || !(fabs(rq.w) <= T(2));
+#pragma unroll
+        for (int t = 1; t < NT; ++t) odd = odd || !plain(ct[t - 1].x) || !plain(ct[t - 1].y);
+        uint64_t left = __ballot(lane < nb && odd);
+        if (left && odd) {
+            rq.x = rq.y = T(0);
+            if (!(fabs(rq.z) <= T(2))) rq.z = T(0);
+            if (!(fabs(rq.w) <= T(2))) rq.w = T(0);
+#pragma unroll
+            for (int t = 1; t < NT; ++t) ct[t - 1] = Pair<T>{T(0), T(0)};
+        }
+        if (lane < nb) {
+            const int v0 = Sh::kGuard + lane * S;
+            stage_weights<T, NS>(cf, beta, horner, rq.z, lds.kx + v0);
+            stage_weights<T, NS>(cf, beta, horner, rq.w, lds.ky + v0);
+        }
+        // rolling: the batch window by window (its points come in row order)
+        for (int done = 0;;) {
+            // opaque: what follows from the key and the lane is computed in every window,
+            // or it would be computed ahead and spilled
+            unsigned key = pkey;
+            int ln = lane;
+            if constexpr (ROLL) asm volatile("" : "+v"(key), "+v"(ln));
+            const int X = (int)(key & ((1u << kStripKeyShift) - 1));
+            const int Y = (int)((int64_t)(key >> kStripKeyShift) - rowbase) - r0;
+            uint64_t in = nb < kStripLanes ? (uint64_t(1) << nb) - 1 : ~uint64_t(0);
+            if constexpr (ROLL) in &= __ballot(Y < top + 16) & (~uint64_t(0) << done);
+            const int count = ROLL ? __popcll(in) : nb;
+            if (!ROLL || in) {
+                // this lane's slot, and the groups of four of every frame
+                constexpr int kBits = Sh::kNarrow ? 3 : 2;
+                const unsigned frame = (unsigned)X >> Sh::kFrameShift;
+                uint64_t bit[kBits], same = in;
+#pragma unroll
+                for (int b = 0; b < kBits; ++b) {
+                    const bool one = (frame >> b) & 1;
+                    bit[b] = __ballot(one);
+                    same &= one ? bit[b] : ~bit[b];
+                }
+                int groups[NF];
+                uint64_t starts = 0;  // first group of every frame, 5 bits each
+                int base = 0;
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    uint64_t m = in;
+#pragma unroll
+                    for (int b = 0; b < kBits; ++b) m &= (f >> b) & 1 ? bit[b] : ~bit[b];
+                    starts |= (uint64_t)base << (5 * f);
+                    groups[f] = (__popcll(m) + 3) >> 2;
+                    base += groups[f];
+                }
+                const int slot = 4 * (int)((starts >> (5 * frame)) & 31) +
+                                 (int)__builtin_amdgcn_mbcnt_hi(
+                                     (unsigned)(same >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((unsigned)same, 0u));
+                // the row tiles these points reach (a rolling window: 32 rows from
+                // `top`, row y in place y mod 32)
+                bool low = true, high = false;
+                if constexpr (ROLL) {
+                    const bool both = __builtin_amdgcn_readlane(Y, done + count - 1) + NS > top + 16;
+                    low = both || !(top & 16);
+                    high = both || (top & 16);
+                } else if constexpr (RT > 1) {
+                    low = __builtin_amdgcn_readfirstlane(Y) < 16;
+                    high = __builtin_amdgcn_readlane(Y, nb - 1) + NS > 16;
+                }
+                // (a wave's LDS writes land in order: the empty slots before the filled)
+                lds.slot[ln] = none;
+                if (ln + kStripLanes < Sh::kSlots) lds.slot[ln + kStripLanes] = none;
+                if ((in >> ln) & 1) {
+                    const int v0 = Sh::kGuard + ln * S;
+                    const int ox = X & ((1 << Sh::kFrameShift) - 1);
+                    StripSlot<T, NT> me;
+                    me.c[0] = Pair<T>{rq.x, rq.y};
+#pragma unroll
+                    for (int t = 1; t < NT; ++t) me.c[t] = ct[t - 1];
+                    // narrow: byte offsets of where row 0 of the tile / column 0 of the frame
+                    // lie in the staged values; wide: the first row, and lane and column
+                    me.at = Sh::kNarrow
+                                ? (unsigned)((v0 - Y) * sizeof(T)) << 16 | (unsigned)((v0 - ox) * sizeof(T))
+                                : (unsigned)(ROLL ? Y & 31 : Y) << 16 | (unsigned)(ln << 4) | (unsigned)ox;
+                    lds.slot[slot] = me;
+                }
+                wave_sync();
+                // operands of the four points from slot 4 n: lane (i16, g) reads point g's
+                constexpr int NB = Sh::kNarrow ? 1 : 2;
+                struct Operands {
+                    T y[RT], x[NB];
+                    Pair<T> c[NT];
+                };
+                const StripSlot<T, NT> *next = lds.slot + g;
+                auto fetch = [&] {
+                    Operands o;
+                    const StripSlot<T, NT> s = *next;
+                    next += 4;
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) o.c[t] = s.c[t];
+                    if constexpr (Sh::kNarrow) {
+                        // both halves at once (neither overflows)
+                        const unsigned at = s.at + (unsigned)(i16 * sizeof(T)) * 0x10001u;
+                        o.y[0] = *reinterpret_cast<const T *>(
+                            reinterpret_cast<const char *>(lds.ky) + (at >> 16));
+                        o.x[0] = *reinterpret_cast<const T *>(
+                            reinterpret_cast<const char *>(lds.kx) + (at & 0xffffu));
+                    } else {
+                        const int ya = (int)(s.at >> 16), xa = (int)(s.at & 15u);
+                        const int v0 = (int)(s.at >> 4 & 63u) * S;
+#pragma unroll
+                        for (int h = 0; h < RT; ++h) {
+                            const int e = (i16 + 16 * h - ya) & (ROLL ? 31 : ~0);
+                            const T v = lds.ky[v0 + (unsigned(e) < NS ? e : 0)];
+                            o.y[h] = unsigned(e) < NS ? v : T(0);
+                        }
+#pragma unroll
+                        for (int h = 0; h < NB; ++h) {
+                            const int e = i16 + 16 * h - xa;
+                            const T v = lds.kx[v0 + (unsigned(e) < NS ? e : 0)];
+                            o.x[h] = unsigned(e) < NS ? v : T(0);
+                        }
+                    }
+                    return o;
+                };
+                Operands cur = fetch();
+                // frames as compile-time constants, so that the accumulators are separate
+                // registers to the compiler (as one array it copies it between frames)
+                unroll<NF>([&](auto fc) {
+                    constexpr int f = decltype(fc)::value;
+                    for (int n = groups[f]; n > 0; --n) {
+                        const Operands o = cur;
+                        cur = fetch();
+                        unroll<RT>([&](auto hc) {
+                            constexpr int h = decltype(hc)::value;
+                            if (RT > 1 && !(h == 0 ? low : high)) return;
+                            const T y = o.y[h];
+                            unroll<NT>([&](auto tc) {
+                                constexpr int t = decltype(tc)::value;
+                                const T ar = y * o.c[t].x, ai = y * o.c[t].y;
+                                re[t][h][f] = M::mul(ar, o.x[0], re[t][h][f]);
+                                im[t][h][f] = M::mul(ai, o.x[0], im[t][h][f]);
+                                if constexpr (NB > 1 && f + 1 < NF) {
+                                    // (no point of the last frame leaves it)
+                                    re[t][h][f + 1] = M::mul(ar, o.x[NB - 1], re[t][h][f + 1]);
+                                    im[t][h][f + 1] = M::mul(ai, o.x[NB - 1], im[t][h][f + 1]);
+                                }
+                            });
+                        });
+                    }
+                });
+                for (uint64_t m = left & in; m; m &= m - 1) {
+                    const int q = __builtin_ctzll(m);
+                    const unsigned key = pts.key[bb + q];
+                    const int i = pts.idx[bb + q];
+                    const Quad<T> p = point_record(pts, i);
+                    const int qx = (int)(key & ((1u << kStripKeyShift) - 1));
+                    const int qy = (int)((int64_t)(key >> kStripKeyShift) - rowbase) - r0;
+                    // (a weight of NaN where the coordinate is)
+                    const T u = (fabs(p.z) <= T(2) ? T(0) : p.z - p.z) + (fabs(p.w) <= T(2) ? T(0) : p.w - p.w);
+                    unroll<NT>([&](auto tc) {
+                        constexpr int t = decltype(tc)::value;
+                        Pair<T> c{p.x, p.y};
+                        if constexpr (t > 0)
+                            c = reinterpret_cast<const Pair<T> *>(pts.c + t * pts.c_tstride)[i - pts.idx_off];
+                        unroll<RT * NF * 4>([&](auto ec) {
+                            constexpr int e = decltype(ec)::value, h = e / (NF * 4), f = e / 4 % NF,
+                                          r = e % 4;
+                            const int dy = (16 * h + M::row(r, g) - qy) & (ROLL ? 31 : ~0);
+                            const int dx = (f << Sh::kFrameShift) + i16 - qx;
+                            if (unsigned(dy) < NS && unsigned(dx) < NS &&
+                                (!Sh::kNarrow || f == qx >> Sh::kFrameShift)) {
+                                const int v0 = Sh::kGuard + q * S;
+                                const T w = lds.kx[v0 + dx] * lds.ky[v0 + dy] + u;
+                                re[t][h][f][r] += c.x * w;
+                                im[t][h][f][r] += c.y * w;
+                            }
+                        });
+                    });
+                }
+                wave_sync();
+            }
+            if constexpr (!ROLL) break;
+            done += count;
+            if (done == nb) break;
+            flush();
+        }
+    }
+    if constexpr (ROLL) {
+        while (top < rows_tile) flush();
+    } else if constexpr (W == 1) {
+        unroll<NT * RT * 16>([&](auto ec) {
+            constexpr int e = decltype(ec)::value;
+            store(e, 16 * (e / 16 % RT) + M::row(e % 4, g), i16, value(ec));
+        });
     } else {
         // eight values of every lane at a time through the staging areas; wave w
         // adds up values w, w + W, ...
@@ -545,7 +616,7 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
                     v.x += x.x;
                     v.y += x.y;
                 }
-                store(e0 + e + wave, v);
+                store(e0 + e + wave, 16 * ((e0 + e + wave) / 16 % RT) + M::row((e0 + e + wave) % 4, g), i16, v);
             }
             __syncthreads();
         });
@@ -1081,7 +1152,7 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
     JFA_DISPATCH_NS(sg.ns, {
         if (phases & kStripSpread) {
             auto kernel = waves > 1 ? spread_strip_kernel<T, NS_, kPieceWaves, false>
-                          : tall    ? spread_strip_kernel<T, NS_, 1, (NS_ <= 8)>
+                          : tall    ? spread_strip_kernel<T, NS_, 1, true>
                                     : spread_strip_kernel<T, NS_, 1, false>;
             kernel<<<dim3(grid, ntr), kStripLanes * waves, 0, stream>>>(
                 sg, pts, bin_start, piece_start, npieces, piece_unit, coef, b, kerevalmeth,
@@ -1139,7 +1210,7 @@ int launch_ragged_strip(const RaggedLaunch &rl, const StripPts<T> &pts, const T 
     const T b = (T)beta;
     JFA_DISPATCH_NS(rl.ns, {
         if (phases & kStripSpread) {
-            auto kernel = rl.tall ? ragged_strip_kernel<T, NS_, (NS_ <= 8)>
+            auto kernel = rl.tall ? ragged_strip_kernel<T, NS_, true>
                                   : ragged_strip_kernel<T, NS_, false>;
             kernel<<<grid, kStripLanes * kRaggedWaves, 0, stream>>>(
                 rl.virt, rl.unit_virt, pts, rl.bin_start, rl.piece_start, rl.npieces,

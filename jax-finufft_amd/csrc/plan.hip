@@ -236,14 +236,21 @@ void jfa::strip_set_rows(StripGeom &sg, int64_t rows) {
 // 37,000 of 64 272 / 274 and 423 / 427; 8208 of 12 51 / 44 and 76 / 64, of 36 56 / 61 and
 // 84 / 86; 1335 of 30 27 / 34 and 31 / 43.  Below two points most short units are empty
 // and write nothing (ns = 3 in fp64, 37,000 of one 160 / 197).
-bool jfa::strip_tall(double points, double units) {
+//
+// ns > 8: short units' tiles are 2.1 (ns = 9) to 2.5 cells per cell, those of 128 rows 1.2
+// to 1.5, at the cost of a slower walk.  60,000 units of 17 points at ns = 12 1159 / 1053
+// us, 33,000 of 31 651 / 689; 81,000 of 12 at ns = 16 1430 / 1150, 43,000 of 23 844 / 705,
+// 24,500 of 7 417 / 353, 5082 of 4 90 / 108.
+bool jfa::strip_tall(int ns, double points, double units) {
     const double even = points / units;
-    return even >= 2 && even < std::min(64.0, units / 400);
+    if (even < 2) return false;
+    if (ns > 8) return even < 64 && units >= (ns > 13 ? 20000 : 50000);
+    return even < std::min(64.0, units / 400);
 }
 
 void jfa::strip_units(StripGeom &sg, int64_t M, int nb, int rows) {
     strip_set_rows(sg, rows > 0 ? rows : strip_short_rows(sg.ns));
-    if (rows <= 0 && strip_tall((double)M * nb, (double)sg.nunits * nb))
+    if (rows <= 0 && strip_tall(sg.ns, (double)M * nb, (double)sg.nunits * nb))
         strip_set_rows(sg, strip_tall_rows(sg.ns));
 }
 
@@ -276,23 +283,34 @@ struct StripNeed {
 static StripNeed strip_need(jfa_plan p, int64_t M) {
     const size_t real = p->is_double ? 8 : 4;
     const int rows = p->opts.gpu_binsizey;
-    StripGeom low = p->sg, tall = p->sg;
-    strip_set_rows(low, rows > 0 ? rows : strip_short_rows(low.ns));
-    strip_set_rows(tall, rows > 0 ? rows : strip_tall_rows(tall.ns));
-    int64_t more;
-    if (p->opts.gpu_maxsubprobsize > 0) {
-        more = M / p->opts.gpu_maxsubprobsize;
-    } else {
-        const int64_t nb = p->batch;
-        more = std::min(std::min(M / 256, 4096 / nb), std::max<int64_t>(low.nunits / 2, 512 / nb));
-        more = std::max(M / kStripPiece, more + more / 64) + 2;  // (sizes are rounded)
+    const int64_t nb = p->batch;
+    StripNeed n{};
+    int64_t cells = 0;
+    auto add = [&](int64_t height, int64_t most) {
+        StripGeom g = p->sg;
+        strip_set_rows(g, height);
+        int64_t more;
+        if (p->opts.gpu_maxsubprobsize > 0) {
+            more = most / p->opts.gpu_maxsubprobsize + 1;
+        } else {
+            more = std::min(std::min(most / 256, 4096 / nb),
+                            std::max<int64_t>(g.nunits / 2, 512 / nb));
+            more = std::max(most / kStripPiece, more + more / 64) + 2;  // (sizes are rounded)
+        }
+        const int64_t pieces = std::min<int64_t>(g.nunits, most) + more;
+        n.pieces = std::max(n.pieces, pieces);
+        n.heavy = std::max(n.heavy, more + 1);
+        cells = std::max(cells, pieces * strip_tile_cells(g));
+    };
+    add(rows > 0 ? rows : strip_short_rows(p->geom.ns), M);
+    if (rows <= 0) {
+        // tall units, of the counts up to M that they suit
+        StripGeom g = p->sg;
+        strip_set_rows(g, strip_short_rows(g.ns));
+        const int64_t units = g.nunits;
+        if (M >= 2 * units && strip_tall(g.ns, 2.0 * units * nb, (double)units * nb))
+            add(strip_tall_rows(g.ns), std::min(M, 64 * units));
     }
-    StripNeed n;
-    n.pieces = std::min<int64_t>(low.nunits, M) + more;
-    n.heavy = more + 1;
-    const int64_t cells = std::max(n.pieces * strip_tile_cells(low),
-                                   (std::min<int64_t>(tall.nunits, M) + more) *
-                                       strip_tile_cells(tall));
     n.tile_bytes = (size_t)cells * 2 * real;
     n.pack_bytes = (size_t)M * 4 * real;
     return n;

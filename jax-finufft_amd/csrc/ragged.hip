@@ -197,8 +197,12 @@ int layout(jfa_ragged r) {
         r->moff[i + 1] = r->moff[i] + r->npts[i];
         bins += g.nbins;
     }
-    // one height for the batch, whose units share one launch
-    if (r->opts.gpu_binsizey <= 0 && strip_tall(unit_points, units))
+    // One height for the batch, whose units share one launch.  Small grids have few rolling
+    // units (ns > 8), so there have to be many problems: 200 of 1e3 to 1e4 points, one
+    // transform each (100,000 short units) 2.42 / 2.77 ms at ns = 11 with short / tall ones, up
+    // to six each (350,000) 7.52 / 7.15.
+    if (r->opts.gpu_binsizey <= 0 && strip_tall(ns, unit_points, units) &&
+        (ns <= 8 || units >= 200000))
         for (StripGeom &s : sg) strip_set_rows(s, strip_tall_rows(ns));
     r->rl.tall = false;
     for (const StripGeom &s : sg) r->rl.tall = r->rl.tall || s.H > strip_short_rows(ns);

@@ -135,8 +135,8 @@ def clear():
     _lib().jfa_tune_clear()
 
 
-# unit height (rows, at most 33 - width) x piece size for ragged batches; (0, 0) is the
-# default rule
+# unit height (rows, at most 33 - width where that is 25 or more) x piece size for ragged
+# batches; (0, 0) is the default rule
 RAGGED_CANDIDATES = [(0, 0), (16, 0), (32, 0), (0, 2048), (32, 2048), (32, 8192)]
 
 
