@@ -19,7 +19,11 @@
 // transposes and scaling kernels they replace move each intermediate two or
 // three times: modes -> 512^3 grid, 256^3 modes, 1.36 -> 0.73 ms; 360^3 modes ->
 // the kept 720 x 375 x 375 cells of a type-3 inner grid, 1.85 -> 1.13 ms; 2048^2
-// grid -> 1024^2 modes, 46 -> 37 us (fp32).  Those stay for axes beyond 4096.
+// grid -> 1024^2 modes, 46 -> 37 us (fp32).  Those stay for plans with an axis these
+// passes do not run (axis_fft): beyond 4096 cells, or of a length whose smallest radix
+// leaves more threads for 32 bytes of columns than a workgroup has (of the even lengths
+// in fp32 1458, 1944, 2000, 2430, 2500, 2592, 2916, 3000, 3200, 3240, 3456, 3750, 3888,
+// 4000, 4050; in fp64 2700, 3000, 3200, 3240, 3456, 3600, 3750, 3840, 3888, 4000, 4050).
 //
 // One workgroup transforms a tile in LDS: one (or a few) contiguous rows along
 // x, or TC neighbouring columns along y / z (TC complex values are 128 bytes
@@ -485,7 +489,7 @@ int launch_rows(const AxisFft &f, const T *tw, int64_t rows, int64_t n, int mode
 }
 
 // Columns per workgroup: 128 bytes of them when P threads per column and the
-// LDS tile (64 KiB for two or more workgroups per CU; up to 128 KiB for long
+// LDS tile (80 KiB, for two workgroups per CU; up to 144 KiB for the longest
 // axes) allow, 32 bytes at least; fewer too while the launch has under 512
 // workgroups (a 2-byte-per-flop pass needs every CU busy, and such small
 // arrays sit in L2, where short segments cost little).

@@ -44,6 +44,16 @@ def _run(plan, x, c, shape):
     return out
 
 
+@pytest.mark.parametrize("modes", [(40, 16), (300, 31), (20, 24, 18)], ids=str)
+def test_auto_takes_strips_on_narrow_grids(modes):
+    # (what test_gpu_strip_tiles compares there, and cannot ask for by method 3)
+    x = [torch.rand(5000, device="cuda") for _ in modes]
+    plan = Plan(1, modes, iflag=1, eps=1e-5, dtype=torch.complex64)
+    plan.setpts(*x)
+    assert _method(plan) == STRIPS
+    plan.destroy()
+
+
 def test_narrow_grid_memory_is_bounded():
     # 24^3 modes, 48^3 cells, width 8: eight slice points of 64 bytes per point
     plan = Plan(1, (24, 24, 24), iflag=1, eps=1e-6, dtype=torch.complex64)
