@@ -4,12 +4,14 @@ Memory is filled by a tensor of the test; what is left is many times what the ke
 that run need."""
 
 import contextlib
+import gc
 
 import numpy as np
 import pytest
 import torch
 
 from gpu_helpers import cnormal, dev, host, rel_l2, uniform_points
+from jax_finufft_amd import _native
 from jax_finufft_amd._native import Plan
 
 pytestmark = pytest.mark.gpu
@@ -24,10 +26,14 @@ def _method(plan):
 
 @contextlib.contextmanager
 def _memory_left(nbytes):
+    # what earlier tests left behind goes first, or it would be freed meanwhile
+    gc.collect()
+    _native.lib().jfa_cache_clear()
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
-    free, _ = torch.cuda.mem_get_info()
-    filler = torch.empty(max(0, free - nbytes), dtype=torch.uint8, device="cuda")
+    filler = []
+    while (free := torch.cuda.mem_get_info()[0] - nbytes) > (64 << 20):
+        filler.append(torch.empty(free, dtype=torch.uint8, device="cuda"))
     try:
         yield
     finally:
