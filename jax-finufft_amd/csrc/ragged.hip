@@ -197,12 +197,19 @@ int layout(jfa_ragged r) {
         r->moff[i + 1] = r->moff[i] + r->npts[i];
         bins += g.nbins;
     }
-    // One height for the batch, whose units share one launch.  Small grids have few rolling
-    // units (ns > 8), so there have to be many problems: 200 of 1e3 to 1e4 points, one
-    // transform each (100,000 short units) 2.42 / 2.77 ms at ns = 11 with short / tall ones, up
-    // to six each (350,000) 7.52 / 7.15.
+    // One height for the batch, whose units share one launch (a launch for each height:
+    // 28 problems of 1e4 to 3.1e5 points 790 -> 858 us).  Tall units make dense problems'
+    // waves longer, so few of the points may be in such: 6 problems of 1e4 to 6.5e4 points, up
+    // to 8 transforms, 456 / 699 us with short / tall ones, 200 of 1e3 to 1e4 1.60 / 1.44 ms.
+    // Small grids have few rolling units (ns > 8), so there have to be many: 200 of 1e3 to
+    // 1e4 points, one transform each (100,000 short units), 2.42 / 2.77 ms at ns = 11, up to
+    // six each (350,000) 7.52 / 7.15.
+    double dense = 0;  // points of dense problems
+    for (int i = 0; i < np; ++i)
+        if (r->npts[i] > (ns <= 8 ? 64 : 256) * (int64_t)sg[i].nunits)
+            dense += (double)r->npts[i] * r->ntr[i];
     if (r->opts.gpu_binsizey <= 0 && strip_tall(ns, unit_points, units) &&
-        (ns <= 8 || units >= 200000))
+        3 * dense <= unit_points && (ns <= 8 || units >= 200000))
         for (StripGeom &s : sg) strip_set_rows(s, strip_tall_rows(ns));
     r->rl.tall = false;
     for (const StripGeom &s : sg) r->rl.tall = r->rl.tall || s.H > strip_short_rows(ns);
