@@ -159,6 +159,9 @@ int wave_transforms(jfa_ragged r, int i, int t) {
     return (t & 1) ? 0 : (t + 1 < r->ntr[i] ? 2 : 1);
 }
 
+// Rows of the units of sparse batches (layout).
+constexpr int kSparseRows = 16;
+
 // Problem geometry, virtual problems, offsets; host only.
 int layout(jfa_ragged r) {
     const int ns = r->kp.ns;
@@ -198,19 +201,28 @@ int layout(jfa_ragged r) {
         bins += g.nbins;
     }
     // One height for the batch, whose units share one launch (a launch for each height:
-    // 28 problems of 1e4 to 3.1e5 points 790 -> 858 us).  Tall units make dense problems'
-    // waves longer, so few of the points may be in such: 6 problems of 1e4 to 6.5e4 points, up
-    // to 8 transforms, 456 / 699 us with short / tall ones, 200 of 1e3 to 1e4 1.60 / 1.44 ms.
-    // Small grids have few rolling units (ns > 8), so there have to be many: 200 of 1e3 to
-    // 1e4 points, one transform each (100,000 short units), 2.42 / 2.77 ms at ns = 11, up to
-    // six each (350,000) 7.52 / 7.15.
-    double dense = 0;  // points of dense problems
-    for (int i = 0; i < np; ++i)
-        if (r->npts[i] > (ns <= 8 ? 64 : 256) * (int64_t)sg[i].nunits)
-            dense += (double)r->npts[i] * r->ntr[i];
-    if (r->opts.gpu_binsizey <= 0 && strip_tall(ns, unit_points, units) &&
-        3 * dense <= unit_points && (ns <= 8 || units >= 200000))
-        for (StripGeom &s : sg) strip_set_rows(s, strip_tall_rows(ns));
+    // 28 problems of 1e4 to 3.1e5 points 790 -> 858 us).  ns <= 8: 16 rows halve the tiles to
+    // merge, but dense problems' units, taller, end late, so there have to be few points or
+    // many units to level them.  9 / 16 rows in us: 41,466 units of 3 points on the mean 511 /
+    // 498, 10,676 of 34 290 / 366, 44,600 of 34 689 / 774, 56,208 of 52 856 / 992, 68,000 of
+    // 49 988 / 1046, 72,206 of 54 1042 / 1010, 79,952 of 112 1265 / 1336, 89,834 of 64 1285 /
+    // 1182, 98,028 of 126 1576 / 1534, 151,500 of 37 1956 / 1721, 128,558 of 6 1601 / 1441, 111,926 of 186 1938 / 1982 (25 rows: 44,600 of 34 889,
+    // 151,500 of 37 1817, 128,558 of 6 1441).  ns > 8: small grids have few rolling units, so
+    // there have to be many, and few points in dense problems: 200 of 1e3 to 1e4 points, one
+    // transform each (128,558 short units), 2.42 / 2.77 ms at ns = 11, up to six each 7.52 /
+    // 7.15.
+    if (r->opts.gpu_binsizey <= 0 && ns <= 8) {
+        const double line = units < 75000 ? 16 : std::min(units / 1300, 125.0);
+        if (unit_points <= line * units)
+            for (StripGeom &s : sg) strip_set_rows(s, kSparseRows);
+    } else if (r->opts.gpu_binsizey <= 0) {
+        double dense = 0;  // points of dense problems
+        for (int i = 0; i < np; ++i)
+            if (r->npts[i] > 256 * (int64_t)sg[i].nunits)
+                dense += (double)r->npts[i] * r->ntr[i];
+        if (strip_tall(ns, unit_points, units) && 3 * dense <= unit_points && units >= 200000)
+            for (StripGeom &s : sg) strip_set_rows(s, strip_tall_rows(ns));
+    }
     r->rl.tall = false;
     for (const StripGeom &s : sg) r->rl.tall = r->rl.tall || s.H > strip_short_rows(ns);
     r->mtot = r->moff[np];
