@@ -234,7 +234,9 @@ void jfa::strip_set_rows(StripGeom &sg, int64_t rows) {
 // Points of an even short unit, short / tall, spreading + merge, ns = 8: 131,000 units of
 // 8 826 / 543 us in fp32, 1242 / 879 in fp64; 262,000 of 30 1700 / 1349 and 2698 / 2162;
 // 37,000 of 64 272 / 274 and 423 / 427; 8208 of 12 51 / 44 and 76 / 64, of 36 56 / 61 and
-// 84 / 86; 1335 of 30 27 / 34 and 31 / 43.  Below two points most short units are empty
+// 84 / 86; 1335 of 30 27 / 34 and 31 / 43.  Whole 3D calls (each slice's points counted), ns =
+// 5: 5825 of 15 123 / 128, 14,800 of 15 186 / 183, of 40 216 / 226; ns = 4, 14,600 of 32 201 /
+// 220; ns = 8, 15,600 of 24 202 / 185, of 64 237 / 229.  Below two points most short units are empty
 // and write nothing (ns = 3 in fp64, 37,000 of one 160 / 197).
 //
 // ns > 8: short units' tiles are 2.1 (ns = 9) to 2.5 cells per cell, those of 128 rows 1.2
@@ -245,7 +247,7 @@ bool jfa::strip_tall(int ns, double points, double units) {
     const double even = points / units;
     if (even < 2) return false;
     if (ns > 8) return even < 64 && units >= (ns > 13 ? 20000 : 50000);
-    return even < std::min(64.0, units / 400);
+    return even < std::min(64.0, units / 600);
 }
 
 void jfa::strip_units(StripGeom &sg, int64_t M, int nb, int rows) {
