@@ -1139,12 +1139,12 @@ int launch_spread_strip(const StripGeom &sg, const StripPts<T> &pts, const int *
     // the line lies: w = 8 in fp32, one wave / four, uniform points: 737 units of 271 points
     // 21 / 16 us, 2052 of 292 30 / 32, of 585 51 / 46, 8208 of 487 111 / 128, of 1219 276 /
     // 263, 37,120 of 216 217 / 350; normal about the centre: 2052 of 487 58 / 40, 8208 of 365
-    // 91 / 97, of 731 175 / 168.  fp64 kernels hold half as many waves and are bound by their
+    // 91 / 97, of 731 175 / 168; w = 5, 3073 of 375, the whole call 171 / 175.  fp64 kernels hold half as many waves and are bound by their
     // products sooner (w = 8: 2052 of 585 82 / 88, of 1170 153 / 137; 5760 of 417 138 / 156,
     // of 1389 427 / 403; w = 11: 3572 of 560 238 / 283, of 1120 442 / 468).
     const int64_t even = std::min<int64_t>(pts.M / sg.nunits, sg.pmax);
     const int64_t line = std::min<int64_t>(
-        std::max<int64_t>((int64_t)sg.nunits * ntr / (sizeof(T) == 4 ? 9 : 5), 128),
+        std::max<int64_t>((int64_t)sg.nunits * ntr / (sizeof(T) == 4 ? 6 : 5), 128),
         sizeof(T) == 4 ? 700 : sg.ns <= 8 ? 2048 : 1024);
     constexpr int kPieceWaves = 4;
     const bool tall = sg.H > strip_short_rows(sg.ns);
