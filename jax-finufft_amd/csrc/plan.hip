@@ -230,24 +230,30 @@ void jfa::strip_set_rows(StripGeom &sg, int64_t rows) {
 
 // Tall units where the short ones hold few points and are many: a unit writes its whole
 // tile and the merge reads it, 2.0 cells per grid cell in short units of ns = 8, 1.4 in
-// tall ones, whose products cost twice as much per point and whose waves are fewer.
-// Points of an even short unit, short / tall, spreading + merge, ns = 8: 131,000 units of
-// 8 826 / 543 us in fp32, 1242 / 879 in fp64; 262,000 of 30 1700 / 1349 and 2698 / 2162;
-// 37,000 of 64 272 / 274 and 423 / 427; 8208 of 12 51 / 44 and 76 / 64, of 36 56 / 61 and
-// 84 / 86; 1335 of 30 27 / 34 and 31 / 43.  Whole 3D calls (each slice's points counted), ns =
-// 5: 5825 of 15 123 / 128, 14,800 of 15 186 / 183, of 40 216 / 226; ns = 4, 14,600 of 32 201 /
-// 220; ns = 8, 15,600 of 24 202 / 185, of 64 237 / 229.  Below two points most short units are empty
-// and write nothing (ns = 3 in fp64, 37,000 of one 160 / 197).
+// tall ones, whose products cost twice as much per point and whose waves are fewer, which
+// points that crowd make worse.  Points of an even short unit (each slice's counted in 3D),
+// short / tall, ns = 8 in fp32, whole calls, uniform points and normal about the centre:
+// 48,700 units of 3 252 / 234 and 221 / 216 us, of 24 268 / 252 and 246 / 250; 90,000 of 24
+// 602 / 572 and 552 / 558; 16,300 of 3 191 / 177 and 170 / 168, of 24 226 / 214 and 201 / 216;
+// 8200 of 8 123 / 117 and 114 / 131; 3D: 15,600 of 24 202 / 185 and 184 / 194, of 64 237 / 229
+// and 220 / 244; 52,600 of 24 169 / 146 and 129 / 132, of 64 187 / 171 and 160 / 173, of 192
+// 255 / 273 and 251 / 308.  Spreading + merge alone: 131,000 units of 8 826 / 543 us in fp32,
+// 1242 / 879 in fp64; 262,000 of 30 1700 / 1349 and 2698 / 2162.  Below two points most short
+// units are empty and write nothing (ns = 3 in fp64, 37,000 of one 160 / 197).
 //
 // ns > 8: short units' tiles are 2.1 (ns = 9) to 2.5 cells per cell, those of 128 rows 1.2
-// to 1.5, at the cost of a slower walk.  60,000 units of 17 points at ns = 12 1159 / 1053
-// us, 33,000 of 31 651 / 689; 81,000 of 12 at ns = 16 1430 / 1150, 43,000 of 23 844 / 705,
-// 24,500 of 7 417 / 353, 5082 of 4 90 / 108.
+// to 1.5, at the cost of a slower walk.  Spreading + merge, uniform points: 60,000 units of
+// 17 at ns = 12 1159 / 1053 us, 33,000 of 31 651 / 689; 81,000 of 12 at ns = 16 1430 / 1150,
+// 43,000 of 23 844 / 705, 24,500 of 7 417 / 353, 5082 of 4 90 / 108.  Whole fp64 calls,
+// uniform and normal points: ns = 13, 61,500 of 4 1011 / 974 and 888 / 922, ns = 16, 76,800 of
+// 4 1087 / 1009 and 930 / 959, of 12 1108 / 1048 and 979 / 1041; ns = 10, 50,600 of 40 1047 /
+// 1080 and 990 / 1093; 3D, ns = 16, 21,100 of 64 218 / 260 and 202 / 280.
 bool jfa::strip_tall(int ns, double points, double units) {
     const double even = points / units;
     if (even < 2) return false;
-    if (ns > 8) return even < 64 && units >= (ns > 13 ? 20000 : 50000);
-    return even < std::min(64.0, units / 600);
+    if (ns > 13) return units >= 20000 && even < 32;
+    if (ns > 8) return units >= 80000 && even < 24;
+    return units >= 12000 && even < std::min(64.0, units / 1500);
 }
 
 void jfa::strip_units(StripGeom &sg, int64_t M, int nb, int rows) {
