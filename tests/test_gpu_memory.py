@@ -31,9 +31,19 @@ def _memory_left(nbytes):
     _native.lib().jfa_cache_clear()
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
+    # (the driver may hold more than it reports as free, so the last of it is found by
+    # asking for it)
+    chunk = 64 << 20
     filler = []
-    while (free := torch.cuda.mem_get_info()[0] - nbytes) > (64 << 20):
+    if (free := torch.cuda.mem_get_info()[0] - nbytes) > 0:
         filler.append(torch.empty(free, dtype=torch.uint8, device="cuda"))
+    last = []
+    with contextlib.suppress(torch.cuda.OutOfMemoryError):
+        while len(last) < 16 * nbytes // chunk:
+            last.append(torch.empty(chunk, dtype=torch.uint8, device="cuda"))
+    filler += last[nbytes // chunk:]
+    del last
+    torch.cuda.empty_cache()
     try:
         yield
     finally:
