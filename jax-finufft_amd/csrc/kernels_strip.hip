@@ -10,9 +10,11 @@
 // columns; strip s owns points whose first x-tap l0x lies in
 // [s*SW, (s+1)*SW), so all of their taps fall in the 64 columns
 // [s*SW, s*SW + 64).  Points are sorted by (strip, l0y) (the "y-major" bins
-// set up by the plan).  A strip is cut into units of H consecutive l0y rows.
-// A unit's whole tile, 16 or 32 rows x 64 columns, lives in the registers of the
-// wave that spreads it, as the accumulators of MFMA products.
+// set up by the plan).  A strip is cut into units of H consecutive l0y rows:
+// short ones of 9 rows (ns <= 8) or 33 - ns, on large sparse grids tall ones of
+// 33 - ns (ns <= 8) or up to 128 (strip_tall).  A unit's whole tile, 16 or 32 rows x
+// 64 columns, lives in the registers of the wave that spreads it, as the
+// accumulators of MFMA products; those of 128 rows roll through 32.
 //
 // Spreading is a contraction over points: tile[y][x] += sum_p (c_p ky_p[y])
 // kx_p[x].  strip_piece takes four points at a time as the K dimension of a
@@ -26,13 +28,13 @@
 // other): figures at strip_piece.
 //
 // Output.  A unit's points are cut into pieces of at most `pmax` points (an
-// empty unit has none), one workgroup of one or four waves per piece.  A piece writes its rows with plain
-// coalesced stores into its own scratch tile of (H + ns - 1) x 64 cells; a
-// merge kernel then writes every fine-grid cell once, as the sum over the
-// units covering it (one to four, up to nine next to a narrow last strip or
-// unit) of their pieces' tiles.  The fine grid is
-// neither zeroed first nor read, no float atomics are used anywhere, and the
-// summation order is fixed, so results are bitwise reproducible.
+// empty unit has none), one workgroup of one or four waves per piece.  A piece
+// writes its rows with plain coalesced stores into its own scratch tile of
+// (H + ns - 1) x 64 cells; a merge kernel then writes every fine-grid cell once,
+// as the sum over the units covering it (one to four, up to nine next to a narrow
+// last strip or unit) of their pieces' tiles.  The fine grid is neither zeroed
+// first nor read, no float atomics are used anywhere, and the summation order is
+// fixed, so results are bitwise reproducible.
 //
 // The same per-piece and per-cell bodies serve one plan (a single problem,
 // blockIdx.y = transform) and a ragged batch of problems (descriptor tables,
@@ -236,23 +238,24 @@ __device__ __forceinline__ PieceRange piece_range(const StripGeom &sg,
 // frames of 16 columns.  ns <= 8: eight frames 8 columns apart, one row tile, so a
 // point adds to exactly one frame: one MFMA each for the real and imaginary parts
 // of four points (half the columns are zeros).  ns > 8, and tall units of ns <= 8
-// (strip_tall): four frames, two row tiles; a point adds to its frame and the next, and to both row tiles where its
-// rows straddle them (batches are in row order, so a row tile no point of the
-// batch touches is skipped).  Each MFMA's four points must share a frame: the
-// points of a batch are ranked by frame (one ballot per bit of the frame) and
-// listed in that order in the slots, every frame's list filled up to a multiple of
-// four with zero strengths; the weights stay where the point's lane wrote them.
+// (strip_tall): four frames, two row tiles; a point adds to its frame and the next,
+// and to both row tiles where its rows straddle them (batches are in row order, so a
+// row tile no point of the batch touches is skipped).  Each MFMA's four points must
+// share a frame: the points of a batch are ranked by frame (one ballot per bit of
+// the frame) and listed in that order in the slots, every frame's list filled up to
+// a multiple of four with zero strengths; the weights stay where the point's lane
+// wrote them.
 //
 // Counted at 1e7 uniform points on 2048^2 (fp32, ns = 8), per point: 19 MFMA
-// cycles, 7.3 VALU wave instructions (of 4 cycles; 104 Horner FMAs over 64 lanes,
+// cycles, 7.1 VALU wave instructions (of 4 cycles; 104 Horner FMAs over 64 lanes,
 // ranking, operand addresses), 7 LDS cycles.  263 us, where adding one point after
 // another to per-lane windows of the tile (10.4 VALU instructions and 9.6 LDS cycles
 // per point) took 268; a unit's points now need no order within a row, which makes
 // the sort's keys 3 bits shorter.  The walk was a chain of LDS reads and adds, so
 // smaller and wider problems gain more: 1e6 fp64 points on 1024^2 cells at ns = 11
-// 275 -> 185 us, 300,007 centre-dense points x 4 transforms on 301 x 255 modes at
-// ns = 6 65 -> 46, 4000 points on 48 x 40 29 -> 11; 2^20 sources of a 3D type 3 at
-// ns = 8 507 -> 314.
+// 275 -> 152 us, 300,007 centre-dense points x 4 transforms on 301 x 255 modes at
+// ns = 6 65 -> 47, 4000 points on 48 x 40 29 -> 8; 2^20 sources of a 3D type 3 at
+// ns = 8 507 -> 320.
 //
 // Tall units of ns > 8 have up to 128 rows, which the accumulators roll over: they hold
 // 32 rows, row y in place y mod 32, and whenever the points move on past the first 16
@@ -626,8 +629,8 @@ __device__ __forceinline__ void strip_piece(const StripGeom &sg, const StripPts<
 // The windows of one axis that reach into window w's first ns - 1 cells from
 // the left: window w - 1, or, for w = 0, the last one or two windows through
 // the periodic wrap (the second when the last window owns fewer than ns - 1
-// cells), w itself among them where the axis is shorter than a window.  Windows start every `step` cells, span `span` and n of them cover
-// nf cells.  Appends (window, offset of w's cell 0 in its tile) to win / off.
+// cells), w itself among them where the axis is shorter than a window.  Windows
+// start every `step` cells, span `span` and n of them cover nf cells.  Appends (window, offset of w's cell 0 in its tile) to win / off.
 __device__ __forceinline__ int left_windows(int w, int step, int span, int n, int64_t nf,
                                             int *win, int *off) {
     int c = 0;
