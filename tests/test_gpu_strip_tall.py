@@ -1,6 +1,7 @@
 """Tall units of the strip spreader (up to 33 - w rows, in 16-column frames; of widths above
-8 up to 128 rows, over which the accumulators roll): asked for through gpu_binsizey on grids of whole and part units, against the plain
-scatter on the same grid, and chosen by the density of a ragged batch and of a plan.
+8 up to 128 rows, over which the accumulators roll): asked for through gpu_binsizey on
+grids of whole and part units, against the plain scatter on the same grid, and chosen by the
+density of a ragged batch and of a plan.
 
 The bound is that of test_gpu_strip_tiles: both add the same terms."""
 
